@@ -1,0 +1,100 @@
+"""Pooled attention and the query-read merge at the edges of their tiles: one,
+two, four and eight waves per workgroup, ragged and empty key prefixes, both
+head dims, values that are not finite, and many-tile query reads, against the
+oracle's formulation in float64."""
+
+import math
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from trifusion_amd.kernels.block import pooled_attention, query_read
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF = torch.bfloat16
+
+
+def attend(q, k, v, mask):
+    s = (q.double() @ k.double().transpose(-1, -2)) / math.sqrt(q.shape[-1])
+    return s.masked_fill(~mask, -math.inf).softmax(-1) @ v.double()
+
+
+def rotated(qkv, cos, sin, heads):
+    b, t, width = qkv.shape
+    d = width // (3 * heads)
+    x = qkv.view(b, t, 3, heads, d).permute(2, 0, 3, 1, 4).float()
+    a, z = x[:2, ..., 0::2], x[:2, ..., 1::2]
+    rot = torch.stack((a * cos - z * sin, a * sin + z * cos), -1).flatten(-2).to(BF)
+    return rot[0], rot[1], x[2]
+
+
+def tables(t, hd):
+    phase = torch.arange(t).float()[:, None] * 10000.0 ** (-torch.arange(0, hd, 2).float() / hd)[None, :]
+    return phase.cos(), phase.sin()
+
+
+@pytest.mark.parametrize("heads,hd", [(3, 64), (2, 32)])
+@pytest.mark.parametrize("t,low", [(1, [1, 0]), (31, [31, 2]), (32, [32, 1]), (33, [33, 32]), (65, [64, 65]),
+                                   (128, [97, 128]), (129, [129, 33]), (451, [451, 257])])
+def test_attention_tiles(t, low, heads, hd):
+    g = torch.Generator().manual_seed(100 * t + hd)
+    low = torch.tensor(low)
+    qkv = (2 * torch.randn(2, t, 3 * heads * hd, generator=g)).to(BF)
+    cos, sin = tables(t, hd)
+    grids = SimpleNamespace(rope_cos=cos.to(DEV), rope_sin=sin.to(DEV), low_lengths=low.to(DEV))
+    y = pooled_attention(qkv.to(DEV), grids, heads).cpu().double()
+    q, k, v = rotated(qkv, cos, sin, heads)
+    mask = (torch.arange(t)[None, :] < low[:, None])[:, None, None, :]
+    some = low > 0
+    ref = attend(q, k, v, mask).transpose(1, 2).reshape(2, t, heads * hd)
+    # half a bf16 step of the result, and fp32 sums of values up to ~8 (scores up
+    # to ~50 in magnitude: relative error of a probability below 50 * 2^-22)
+    err = (y - ref).abs()[some]
+    assert (err <= ref.abs()[some] * 2.0**-8 + 8 * 50 * 2.0**-22).all(), err.max()
+    assert not y[~some].any()
+
+
+def test_attention_infinite_value():
+    """A value row that is not finite reaches the queries that attend to it as in
+    IEEE arithmetic, and a row past the key prefix reaches none."""
+    t, heads, hd = 70, 1, 64
+    g = torch.Generator().manual_seed(5)
+    qkv = torch.randn(2, t, 3 * heads * hd, generator=g).to(BF)
+    qkv[0, 3, 2 * hd + 5] = math.inf
+    qkv[0, 40, 2 * hd + 7] = math.nan
+    qkv[1, 60, 2 * hd :] = math.inf
+    low = torch.tensor([t, 60])
+    cos, sin = tables(t, hd)
+    grids = SimpleNamespace(rope_cos=cos.to(DEV), rope_sin=sin.to(DEV), low_lengths=low.to(DEV))
+    y = pooled_attention(qkv.to(DEV), grids, heads).cpu()
+    assert torch.isposinf(y[0, :, 5]).all() and y[0, :, 7].isnan().all()
+    rest = [i for i in range(hd) if i not in (5, 7)]
+    assert y[0][:, rest].isfinite().all() and y[1].isfinite().all()
+    clean = qkv.clone()
+    clean[0, 3, 2 * hd + 5] = 0
+    clean[0, 40, 2 * hd + 7] = 0
+    clean[1, 60, 2 * hd :] = 0
+    z = pooled_attention(clean.to(DEV), grids, heads).cpu()
+    # the other dims run the fp32 product on the affected tiles: equal up to its rounding
+    assert (y[0][:, rest].float() - z[0][:, rest].float()).abs().max() <= 2.0**-8 * z[0].abs().max()
+    assert torch.equal(y[1], z[1])
+
+
+@pytest.mark.parametrize("t,lengths", [(64, [64, 0]), (520, [513, 1]), (2049, [2049, 700])])
+def test_query_read_merges_many_tiles(t, lengths):
+    g = torch.Generator().manual_seed(t)
+    q = torch.randn(10, 256, generator=g).to(BF)
+    kv = torch.randn(2, t, 512, generator=g).to(BF)
+    lengths = torch.tensor(lengths)
+    y = query_read(q.to(DEV), kv.to(DEV), lengths.to(DEV), 8).cpu().double()
+    k, v = kv.view(2, t, 2, 8, 32).permute(2, 0, 3, 1, 4).unbind(0)
+    qq = q.view(10, 8, 32).transpose(0, 1)[None].expand(2, -1, -1, -1)
+    mask = (torch.arange(t)[None, :] < lengths[:, None])[:, None, None, :]
+    ref = attend(qq, k, v, mask).transpose(1, 2).reshape(2, 10, 256)
+    some = lengths > 0
+    err = (y - ref).abs()[some]
+    # half a bf16 step and fp32 sums of values up to ~5
+    assert (err <= ref.abs()[some] * 2.0**-8 + 5 * 64 * 2.0**-23).all(), err.max()
+    assert not y[~some].any()

@@ -8,8 +8,6 @@
 //                  masking.py:59-67);
 //   glu_depthwise  F.glu -> masked depthwise conv (model.py:73);
 //   norm_silu      RMSNorm of a bf16 row -> SiLU (model.py:74);
-//   attention      rotary q/k (bf16) -> masked fp32 softmax attention ->
-//                  [B, T, H D] bf16 (model.py:84-104, attention.py:8-18);
 //   merge_gate     mean of the two Mamba directions -> RMSNorm (fp32), and the
 //                  3-way gate linear of cat(cn, mn, an) (model.py:180-186);
 //   merge_conv     gated concatenation (fp32) -> masked depthwise conv (bf16)
@@ -17,8 +15,8 @@
 // Arithmetic per element follows the unfused kernels the block otherwise runs
 // (the row norms of elementwise.hip, the depthwise, pooling, rotary and gate
 // kernels of trifusion_block.hip), so outputs match those paths bit for bit
-// except the gate dot product and the attention, whose sums run in another
-// order than the library GEMM and softmax.
+// except the gate dot product, whose sum runs in another order than the
+// library GEMM.
 #include "common.h"
 
 namespace tf {
@@ -441,158 +439,6 @@ __global__ __launch_bounds__(256) void glu_norm_silu_kernel(const uint16_t* __re
   }
 }
 
-// ---- rotary + masked attention on the pooled grid -------------------------------
-// One wave per (tile of 16 queries, head, batch row). Each query belongs to four
-// lanes, each holding a quarter of its head dims; together they walk the valid
-// keys j < low_length with one online softmax, G keys at a time (independent
-// dot products). Keys (rotated and rounded to bf16 like the rotary kernel's
-// output) and values of 64 positions at a time sit in LDS as bf16.
-
-// Rotation of the 8 dims 8 c8 .. 8 c8 + 7 of a row (pairs 4 c8 .. 4 c8 + 3):
-// x1 cos - x2 sin and x1 sin + x2 cos with separate multiplies and adds, rounded
-// to bf16, as the reference's rotary forms them. cs4, sn4: the pairs' cos and
-// sin (16-byte aligned).
-__device__ __forceinline__ void rotate8(const uint16_t* src, const float* cs4, const float* sn4, float (&o)[8]) {
-#pragma clang fp contract(off)
-  float v[8];
-  ld8(src, v);
-  const float4 c = *reinterpret_cast<const float4*>(cs4), n = *reinterpret_cast<const float4*>(sn4);
-  const float co[4] = {c.x, c.y, c.z, c.w}, si[4] = {n.x, n.y, n.z, n.w};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float a = v[2 * e], z = v[2 * e + 1];
-    o[2 * e] = round_bf16(a * co[e] - z * si[e]);
-    o[2 * e + 1] = round_bf16(a * si[e] + z * co[e]);
-  }
-}
-
-constexpr int kAttSplit = 4;                  // lanes per query
-constexpr int kAttQueries = 64 / kAttSplit;   // queries per wave
-constexpr int kAttGroup = 4;                  // keys scored together
-
-// Lane (qi, part) = (lane % 16, lane / 16) holds dims [part D/4, (part+1) D/4) of
-// query qi's rotated q and of its output; a score is the sum of the four lanes'
-// partial dots (two xor shuffles), so all four keep the same softmax state.
-template <int D>
-__global__ __launch_bounds__(64) void attention_kernel(const uint16_t* __restrict__ qkv, const float* __restrict__ cs,
-                                                       const float* __restrict__ sn,
-                                                       const int64_t* __restrict__ low_lengths,
-                                                       uint16_t* __restrict__ y, int LT, int H, float scale) {
-  constexpr int RS = D + 8;  // LDS row stride (bf16 elements; rows stay 16-byte aligned)
-  constexpr int DP = D / kAttSplit;  // dims per lane
-  // the rotated keys and the values are bf16 numbers, so bf16 storage is exact
-  __shared__ __align__(16) uint16_t ks[64 * RS];
-  __shared__ __align__(16) uint16_t vs[64 * RS];
-  const int lane = threadIdx.x;
-  const int qi = lane % kAttQueries, part = lane / kAttQueries;
-  const int t = blockIdx.x * kAttQueries + qi, h = blockIdx.y, b = blockIdx.z;
-  const int LL = clamp_len(low_lengths, b, LT);
-  const int64_t width = static_cast<int64_t>(3) * H * D;
-  constexpr int G8 = D / 8;  // 8-dim groups per row
-  // the lane's own dims of its query, rotated (groups part DP / 8 ..)
-  float q[DP];
-  {
-    const int tq = t < LT ? t : 0;
-    const uint16_t* qrow = qkv + (static_cast<int64_t>(b) * LT + tq) * width + static_cast<int64_t>(h) * D;
-#pragma unroll
-    for (int gi = 0; gi < DP / 8; ++gi) {
-      const int c8 = part * (DP / 8) + gi;
-      float o[8];
-      rotate8(qrow + 8 * c8, cs + static_cast<int64_t>(tq) * (D / 2) + 4 * c8,
-              sn + static_cast<int64_t>(tq) * (D / 2) + 4 * c8, o);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) q[8 * gi + e] = o[e];
-    }
-  }
-  float acc[DP];
-#pragma unroll
-  for (int i = 0; i < DP; ++i) acc[i] = 0.f;
-  float m = -INFINITY, l = 0.f;
-  for (int j0 = 0; j0 < LL; j0 += 64) {
-    const int nk = min(64, LL - j0);
-    // stage the tile's keys (rotated) and values: task (row r, group c8) per
-    // lane, G8 lanes per row, so a load instruction reads whole 128-byte rows.
-    // Rows past the tile's keys repeat its last key (never read by the scores).
-#pragma unroll
-    for (int it = 0; it < G8; ++it) {
-      const int idx = lane + 64 * it, r = idx / G8, c8 = idx % G8;
-      const int j = j0 + min(r, nk - 1);
-      const uint16_t* row = qkv + (static_cast<int64_t>(b) * LT + j) * width + static_cast<int64_t>(h) * D;
-      float o[8];
-      rotate8(row + static_cast<int64_t>(H) * D + 8 * c8, cs + static_cast<int64_t>(j) * (D / 2) + 4 * c8,
-              sn + static_cast<int64_t>(j) * (D / 2) + 4 * c8, o);
-      st8_bf16(ks + r * RS + 8 * c8, o);
-      *reinterpret_cast<uint4*>(vs + r * RS + 8 * c8) =
-          *reinterpret_cast<const uint4*>(row + static_cast<int64_t>(2) * H * D + 8 * c8);
-    }
-    __syncthreads();
-    const uint16_t* kp = ks + part * DP;
-    const uint16_t* vp = vs + part * DP;
-    for (int jb = 0; jb < nk; jb += kAttGroup) {
-      float sc[kAttGroup];
-#pragma unroll
-      for (int g = 0; g < kAttGroup; ++g) {
-        const int jj = jb + g < nk ? jb + g : 0;
-        float part_dot = 0.f;
-#pragma unroll
-        for (int i = 0; i < DP; i += 8) {
-          float kv[8];
-          ld8(kp + jj * RS + i, kv);
-#pragma unroll
-          for (int e = 0; e < 8; e += 2) part_dot += q[i + e] * kv[e] + q[i + e + 1] * kv[e + 1];
-        }
-        sc[g] = part_dot;
-      }
-#pragma unroll
-      for (int g = 0; g < kAttGroup; ++g) {
-        sc[g] += __shfl_xor(sc[g], kAttQueries, 64);
-        sc[g] += __shfl_xor(sc[g], 2 * kAttQueries, 64);
-      }
-      float mx = m;
-#pragma unroll
-      for (int g = 0; g < kAttGroup; ++g) {
-        sc[g] = jb + g < nk ? sc[g] * scale : -INFINITY;
-        mx = fmaxf(mx, sc[g]);
-      }
-      const float corr = expf(m - mx);
-      float pr[kAttGroup];
-      float psum = 0.f;
-#pragma unroll
-      for (int g = 0; g < kAttGroup; ++g) {
-        pr[g] = expf(sc[g] - mx);
-        psum += pr[g];
-      }
-      l = l * corr + psum;
-#pragma unroll
-      for (int i = 0; i < DP; ++i) acc[i] *= corr;
-#pragma unroll
-      for (int g = 0; g < kAttGroup; ++g) {
-        const int jj = jb + g < nk ? jb + g : 0;
-#pragma unroll
-        for (int i = 0; i < DP; i += 8) {
-          float vv[8];
-          ld8(vp + jj * RS + i, vv);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[i + e] += pr[g] * vv[e];
-        }
-      }
-      m = mx;
-    }
-    __syncthreads();
-  }
-  if (t < LT) {
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
-    uint16_t* dst = y + (static_cast<int64_t>(b) * LT + t) * H * D + static_cast<int64_t>(h) * D + part * DP;
-#pragma unroll
-    for (int i = 0; i < DP; i += 8) {
-      float o[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = acc[i + e] * inv;
-      st8_bf16(dst + i, o);
-    }
-  }
-}
-
 // ---- mean of the two directions -> RMSNorm, and the 3-way gate ------------------
 // One wave per row: mn = rms((mf + mb) / 2) w as the mean row norm computes it
 // (fp32 out), then g_j = bf16(sum_c bf16(s_c) W[j, c] + bias_j) over
@@ -876,31 +722,6 @@ extern "C" int tf_glu_depthwise(const void* up, const void* w, const void* bias,
   }
   TF_GLU(3) TF_GLU(7)
 #undef TF_GLU
-  return TF_ERR_SHAPE;
-}
-
-extern "C" int tf_pooled_attention(const void* qkv, const float* cos_t, const float* sin_t,
-                                   const int64_t* low_lengths, void* y, int64_t batch, int64_t low_time,
-                                   int64_t heads, int64_t head_dim, void* stream) {
-  if (!qkv || !cos_t || !sin_t || !low_lengths || !y) return TF_ERR_NULL;
-  if (batch < 0 || low_time < 0 || heads < 1 || heads > 65535 || batch > 65535 || batch * low_time > 0x7fffffff)
-    return TF_ERR_SHAPE;
-  // the tables are read 4 pairs (16 bytes) at a time
-  if (!tf::a16(qkv) || !tf::a16(y) || !tf::a16(cos_t) || !tf::a16(sin_t)) return TF_ERR_SHAPE;
-  if (batch * low_time == 0) return TF_OK;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(static_cast<uint32_t>((low_time + tf::kAttQueries - 1) / tf::kAttQueries),
-                  static_cast<uint32_t>(heads), static_cast<uint32_t>(batch));
-  const float scale = 1.0f / sqrtf(static_cast<float>(head_dim));
-#define TF_ATT(DV)                                                                                                \
-  if (head_dim == DV) {                                                                                            \
-    hipLaunchKernelGGL(tf::attention_kernel<DV>, grid, dim3(64), 0, s, static_cast<const uint16_t*>(qkv), cos_t,   \
-                       sin_t, low_lengths, static_cast<uint16_t*>(y), static_cast<int>(low_time),                  \
-                       static_cast<int>(heads), scale);                                                            \
-    return tf::launch_status();                                                                                    \
-  }
-  TF_ATT(32) TF_ATT(64)
-#undef TF_ATT
   return TF_ERR_SHAPE;
 }
 

@@ -183,6 +183,56 @@ __device__ __forceinline__ u32x4 load_row8(const uint16_t* row, int k0) {
   return r;
 }
 
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// Element offset of 8-byte unit u (0..15) of row t (0..63) in a [64][64] bf16
+// row buffer. Units are XOR-swizzled by the row, so that the access patterns
+// each touch 16 distinct units (all 32 banks once) per 16 lanes: row-form
+// reads (16 rows, one unit), transposing reads (4 rows x 4 units) and the
+// rotary's row writes (rows t and t + 4, units 2 ng (+1) of ng = 0..7: bit 0
+// of the swizzle differs between the two rows, so one writes even units and
+// the other odd ones).
+__device__ __forceinline__ int rb_off(int t, int u) {
+  const int swz = ((t & 3) << 2) | ((t >> 2) & 3);
+  return t * 64 + ((u ^ swz) << 2);
+}
+
+__device__ __forceinline__ u32x2 rb_read(const uint16_t* buf, int t, int u) {
+  return *reinterpret_cast<const u32x2*>(buf + rb_off(t, u));
+}
+
+// Row-form MFMA operand of k-step s (contraction over the 64 columns) of row t:
+// slots j hold columns kidx(s, hh, j).
+__device__ __forceinline__ u32x4 row_operand(const uint16_t* buf, int t, int s, int hh) {
+  const int u = 8 * (s >> 1) + 4 * (s & 1) + hh;
+  const u32x2 lo = rb_read(buf, t, u), hi = rb_read(buf, t, u + 2);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// Transposed MFMA operand of k-step s (contraction over the 64 rows) for the
+// 32 columns of column tile `tile`: lane (c32, hh) receives column
+// 32 tile + c32 at rows kidx(s, hh, j). Within each 16-lane group the source
+// lane i = 4k + c reads row r0 + k, unit u0 + c, and the transposing read
+// hands output lane j column 4 u0 + j of rows r0 .. r0 + 3.
+__device__ __forceinline__ u32x4 tr_operand(const uint16_t* buf, int tile, int s, int lane) {
+  const int g = lane >> 4;
+  const int i = lane & 15;
+  const int r0 = 32 * (s >> 1) + 16 * (s & 1) + 4 * (g >> 1) + (i >> 2);
+  const int u = 8 * tile + 4 * (g & 1) + (i & 3);
+  const uint16_t* p0 = buf + rb_off(r0, u);
+  const uint16_t* p1 = buf + rb_off(r0 + 8, u);
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0));
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p1));
+  const u32x2 ua = __builtin_bit_cast(u32x2, a), ub = __builtin_bit_cast(u32x2, b);
+  return u32x4{ua[0], ua[1], ub[0], ub[1]};
+}
+
+__device__ __forceinline__ void rb_write16(uint16_t* buf, int t, int u, const u32x4& x) {
+  *reinterpret_cast<u32x2*>(buf + rb_off(t, u)) = u32x2{x[0], x[1]};
+  *reinterpret_cast<u32x2*>(buf + rb_off(t, u + 1)) = u32x2{x[2], x[3]};
+}
+
 __device__ __forceinline__ u32x4 as_u4(const float4& f) { return __builtin_bit_cast(u32x4, f); }
 __device__ __forceinline__ float4 as_f4(const u32x4& u) { return __builtin_bit_cast(float4, u); }
 
