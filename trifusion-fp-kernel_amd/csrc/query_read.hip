@@ -93,25 +93,46 @@ __global__ __launch_bounds__(64) void query_read_tiles_kernel(const uint16_t* __
   }
 }
 
-// One thread per (query, dim) of one (head, batch row): merge the S tiles.
+// Merges the S tiles of one (query, head, batch row): eight groups of D threads
+// take the tiles g, g + 8, ..., and their sums are added in group order. (One
+// thread per (query, dim) walking all S tiles was a chain of dependent loads: the
+// whole read of a 72 s file's fine grid, 451 tiles, took 254 us, now 55.)
+constexpr int kMergeGroups = 8;
+
 template <int NQ, int D>
-__global__ __launch_bounds__(NQ * D) void query_read_merge_kernel(const float* __restrict__ part,
-                                                                  uint16_t* __restrict__ y, int H, int S) {
-  const int h = blockIdx.x, b = blockIdx.y;
-  const int qi = threadIdx.x / D, d = threadIdx.x - qi * D;
-  const float* base = part + (static_cast<int64_t>(b) * H + h) * S * rec_floats<D>(NQ) + qi * (D + 2);
+__global__ __launch_bounds__(kMergeGroups * D) void query_read_merge_kernel(const float* __restrict__ part,
+                                                                            uint16_t* __restrict__ y, int H, int S) {
+  constexpr int R = rec_floats<D>(NQ);
+  __shared__ float top[kMergeGroups * D / 64];
+  __shared__ float sum[kMergeGroups][D + 1];
+  const int qi = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x, grp = tid / D, d = tid % D;
+  const float* base = part + (static_cast<int64_t>(b) * H + h) * S * R + qi * (D + 2);
   float m = -INFINITY;
-  for (int s = 0; s < S; ++s) m = fmaxf(m, base[s * rec_floats<D>(NQ)]);
+  for (int s = tid; s < S; s += kMergeGroups * D) m = fmaxf(m, base[static_cast<int64_t>(s) * R]);
+  m = wave_max(m);
+  if ((tid & 63) == 0) top[tid >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kMergeGroups * D / 64; ++i) m = fmaxf(m, top[i]);
   float l = 0.f, o = 0.f;
   if (m != -INFINITY) {
-    for (int s = 0; s < S; ++s) {
-      const float* r = base + s * rec_floats<D>(NQ);
+#pragma unroll 4
+    for (int s = grp; s < S; s += kMergeGroups) {
+      const float* r = base + static_cast<int64_t>(s) * R;
       const float w = r[0] == -INFINITY ? 0.f : expf(r[0] - m);
       l += w * r[1];
       o += w * r[2 + d];
     }
   }
-  y[(static_cast<int64_t>(b) * NQ + qi) * H * D + h * D + d] = f32_to_bf16(l > 0.f ? o / l : 0.f);
+  sum[grp][d] = o;
+  if (d == 0) sum[grp][D] = l;
+  __syncthreads();
+  if (grp == 0) {
+#pragma unroll
+    for (int g = 1; g < kMergeGroups; ++g) o += sum[g][d], l += sum[g][D];
+    y[(static_cast<int64_t>(b) * NQ + qi) * H * D + h * D + d] = f32_to_bf16(l > 0.f ? o / l : 0.f);
+  }
 }
 
 }  // namespace
@@ -145,7 +166,7 @@ extern "C" int tf_query_read(const void* q, const void* kv, const int64_t* key_l
                      part, static_cast<int>(time), static_cast<int>(heads), tiles, scale);
   if (const int rc = tf::launch_status()) return rc;
   hipLaunchKernelGGL((tf::query_read_merge_kernel<10, 32>),
-                     dim3(static_cast<uint32_t>(heads), static_cast<uint32_t>(batch)), dim3(10 * 32), 0, s, part,
-                     static_cast<uint16_t*>(y), static_cast<int>(heads), tiles);
+                     dim3(10, static_cast<uint32_t>(heads), static_cast<uint32_t>(batch)),
+                     dim3(tf::kMergeGroups * 32), 0, s, part, static_cast<uint16_t*>(y), static_cast<int>(heads), tiles);
   return tf::launch_status();
 }
