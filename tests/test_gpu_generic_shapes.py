@@ -1,0 +1,91 @@
+"""The generic recurrence kernel at the edges of its tiles: state dims that are
+not a multiple of 32 (through the C ABI, which takes any even N <= 128 and any
+P <= 64), strides it cannot read four elements at a time, every dtype, ragged
+lengths, both directions, and values that are not finite."""
+
+import ctypes
+import math
+
+import pytest
+import torch
+
+from oracle.recurrence import fused_mamba_chunked, fused_mamba_f64, fused_mamba_reversed, max_rel
+from trifusion_amd import _lib
+from trifusion_amd.mamba_fused import fused_mamba
+from trifusion_amd.synthetic import clip_inputs
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def call(args, out, lengths=None, reverse=False):
+    """The C entry directly: the Python wrapper takes only N and P of the model."""
+    q, k, v, adt, dt, trap, qb, kb, angles, d, z = args
+    a = _lib.MambaArgs()
+    for name, t in (("q", q), ("k", k), ("v", v), ("adt", adt), ("dt", dt), ("trap", trap), ("angles", angles),
+                    ("z", z), ("out", out)):
+        setattr(a, name, t.data_ptr())
+        setattr(a, name + "_dtype", _lib.dtype_code(t, "test"))
+        getattr(a, name + "_stride")[:] = t.stride()
+    a.qb, a.kb, a.d = qb.data_ptr(), kb.data_ptr(), d.data_ptr()
+    a.lengths = None if lengths is None else lengths.data_ptr()
+    a.batch, a.time, a.heads, a.head_dim = v.shape
+    a.qk_heads, a.state, a.rotary = q.shape[2], q.shape[3], angles.shape[3]
+    a.variant, a.reverse = _lib.VARIANTS["generic"], int(reverse)
+    _lib.check(_lib.load().tf_fused_mamba(ctypes.byref(a), _lib.stream_of(v)), "fused_mamba")
+    return out
+
+
+def on(args):
+    return tuple(x.to(DEV) for x in args)
+
+
+@pytest.mark.parametrize("n,p,r", [(2, 1, 1), (6, 5, 3), (18, 33, 9), (32, 32, 16), (34, 64, 17), (66, 63, 20),
+                                   (96, 32, 24), (98, 64, 49), (128, 64, 64)])
+@pytest.mark.parametrize("t", [1, 64, 97])
+def test_shapes_against_float64(n, p, r, t):
+    args = clip_inputs(2, t, heads=2, head_dim=p, state=n, rotary=r, dtype=torch.float32, seed=n + t)
+    out = torch.full((2, t, 2, p), math.nan, device=DEV)
+    call(on(args), out)
+    ref = fused_mamba_f64(*args)
+    # 32-bit sums of up to 128 + 64 terms; the walk carries them over two chunks
+    assert max_rel(out.cpu(), ref) <= 5e-6
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_lengths_and_strides(dtype, reverse):
+    args = clip_inputs(5, 130, heads=4, head_dim=64, state=64, dtype=dtype, ctrl_dtype=torch.float32, qk_heads=2,
+                       seed=3)
+    lengths = torch.tensor([130, 0, 1, 33, 64])
+    # rows of every operand at odd offsets and strides: no four-element loads
+    odd = []
+    for i, x in enumerate(on(args)):
+        if i in (0, 1, 2, 10):
+            wide = torch.full((*x.shape[:-1], x.shape[-1] + 3), math.nan, device=DEV, dtype=x.dtype)
+            wide[..., 1 : 1 + x.shape[-1]] = x
+            x = wide[..., 1 : 1 + x.shape[-1]]
+        odd.append(x)
+    even = torch.full((5, 130, 4, 64), math.nan, device=DEV)
+    strided = torch.full((5, 130, 4, 65), math.nan, device=DEV)[..., 1:]
+    call(on(args), even, lengths.to(DEV), reverse)
+    call(tuple(odd), strided, lengths.to(DEV), reverse)
+    assert torch.equal(even, strided)  # the same arithmetic whatever the loads
+    ref = (fused_mamba_reversed if reverse else fused_mamba_chunked)(*args, lengths=lengths)
+    assert max_rel(even.cpu(), ref) <= (1e-5 if dtype == torch.float32 else 1e-3)
+    for i, length in enumerate(lengths.tolist()):
+        assert not even[i, length:].any()
+
+
+def test_infinite_value_is_causal():
+    """A row of v that is not finite leaves every earlier row as it was."""
+    args = on(clip_inputs(1, 100, heads=1, head_dim=64, state=64, dtype=torch.float32, seed=9))
+    clean = fused_mamba(*args)
+    for at, bad in ((40, math.inf), (70, math.nan)):
+        v = args[2].clone()
+        v[0, at, 0, 3] = bad
+        y = fused_mamba(*args[:2], v, *args[3:])
+        assert max_rel(y[:, :at].cpu(), clean[:, :at].cpu()) <= 5e-6
+        assert not y[0, at, 0, 3].isfinite() and not y[0, at + 1 :, 0, 3].isfinite().any()
+        rest = [i for i in range(64) if i != 3]
+        assert max_rel(y[..., rest].cpu(), clean[..., rest].cpu()) <= 5e-6
