@@ -19,7 +19,15 @@
 //                32x32 tile of the scores each
 //   products 2   waves 0-3: scores v, gate, store; waves 4-7: state tiles
 // Contractions run on v_mfma_f32_32x32x2_f32: products and sums of full 32-bit
-// operands. N is padded to a multiple of 32 and P to 32 or 64 with zeros in LDS.
+// operands. N is padded to 32, 64 or 128 and P to 32 or 64 with zeros in LDS.
+//
+// What bounds it: the chain of one chunk, ~11 us at N = P = 64 of which the
+// products take ~4 (a SIMD's two waves share a 32-bit matrix unit), the rest
+// being the latency of controls, phase and rotation between barriers. B4 L400
+// H16 P64 N64, fp32: 80 us (2,155 us with contractions formed element by
+// element from LDS and one thread per phase pair); B1 L1600 H16 N128: 446 us
+// (13.2 ms). 32-bit offsets take the clip from 108 to 80 us against 64-bit ones
+// (fewer scalar registers spilled), so they are used wherever they fit.
 #include "mfma_tile.h"
 
 // Outside the contractions every product and sum is rounded on its own, as the
@@ -36,7 +44,6 @@ constexpr int kThreads = 512;
 constexpr int kNMax = 128;
 constexpr int kPMax = 64;
 constexpr int kRowLanes = 8;                // lanes per row in the rotation
-constexpr int kPairsPerWave = kNMax / 2 / 8;  // phase pairs of one wave, at most
 
 // sigmoid with the correctly rounded-to-1-ulp expf rather than the fast
 // hardware exp: the trapezoid weights feed the bf16 rounding of kr.
@@ -65,14 +72,28 @@ __device__ __forceinline__ double tanh_f64(double x) {
   return __builtin_copysign((1.0 - e) * q, x);
 }
 
-// Inclusive fp64 prefix sum over the 64 lanes of the wave.
-__device__ __forceinline__ double wave_scan_f64(double v, int lane) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const double o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
-  }
-  return v;
+// Inclusive fp64 prefix sum over the 64 lanes of the wave on DPP.
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_f64(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint64_t lo = dpp_u32<CTRL, ROW_MASK>(static_cast<uint32_t>(u));
+  const uint64_t hi = dpp_u32<CTRL, ROW_MASK>(static_cast<uint32_t>(u >> 32));
+  return __builtin_bit_cast(double, lo | (hi << 32));
+}
+__device__ __forceinline__ double wave_scan_f64(double x) {
+  x += dpp_f64<kDppRowShr + 1>(x);
+  x += dpp_f64<kDppRowShr + 2>(x);
+  x += dpp_f64<kDppRowShr + 4>(x);
+  x += dpp_f64<kDppRowShr + 8>(x);
+  x += dpp_f64<kDppRowBcast15, 0xa>(x);
+  x += dpp_f64<kDppRowBcast31, 0xc>(x);
+  return x;
+}
+__device__ __forceinline__ double last_lane_f64(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint64_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), 63));
+  const uint64_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), 63));
+  return __builtin_bit_cast(double, lo | (hi << 32));
 }
 
 // Four consecutive elements of a 16- or 32-bit float row at an address that is
@@ -87,7 +108,8 @@ __device__ __forceinline__ float4 load4_f32(const void* p, int dtype, int64_t i)
 }
 
 // Elements n0 .. n0 + 3 of a row (0 past `n`).
-__device__ __forceinline__ float4 load_piece(const void* p, int dtype, int64_t row, int64_t st, int n0, int n, bool vec) {
+template <typename I>
+__device__ __forceinline__ float4 load_piece(const void* p, int dtype, I row, I st, int n0, int n, bool vec) {
   if (vec) return n0 < n ? load4_f32(p, dtype, row + n0) : make_float4(0.f, 0.f, 0.f, 0.f);
   float x[4];
 #pragma unroll
@@ -99,9 +121,15 @@ __device__ __forceinline__ f32x16 mfma_f32(float x, float y, const f32x16& acc) 
   return __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc, 0, 0, 0);
 }
 
-// Rows of q/k (v) can be read four elements at a time.
-struct GenericVec {
-  int q, k, v;
+// Operand block with strides and offsets of type I: 32-bit ones where every
+// offset fits (address arithmetic in one register), else 64-bit ones. A
+// reversed call's time strides are negated; the kernel starts at row L - 1.
+template <typename I>
+struct GenericParams {
+  tf_mamba_args a;
+  I q[4], k[4], v[4], z[4], g[4], o[4];  // [batch, time, head, element]
+  I ad[3], dt[3], tr[3];                 // [batch, head, time]
+  int qvec, kvec, vvec;                  // rows can be read four elements at a time
 };
 
 template <int NT>
@@ -119,23 +147,55 @@ struct GenericShared {
     float trig[kChunk * TS];  // until the rotation
     float sc[kChunk * SS];    // from the products on
   };
+  float qb[NP], kb[NP], qw[NP], kw[NP];  // biases and norm weights, 0 past the state dim
   float cs[kChunk], gamma[kChunk], scale[kChunk], dt[kChunk], wv[kChunk], ecs[kChunk], qk[kChunk];
   int wild;  // the chunk's values hold an infinity or NaN
 };
 
-// NT: 32-channel tiles of the state dim. ROUND: some operand is 16-bit, so the
-// rounding points are not the identity.
-template <int NT, bool ROUND>
-__global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_args a, const GenericVec vec) {
+// 16 elements at offsets off(e) of a float array of any dtype (one branch on
+// the dtype, not one per element).
+template <typename F>
+__device__ __forceinline__ void gather16(const void* p, int dtype, F&& off, float (&x)[16]) {
+  if (dtype == TF_FLOAT32) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] = static_cast<const float*>(p)[off(e)];
+  } else if (dtype == TF_BFLOAT16) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] = bf16_to_f32(static_cast<const uint16_t*>(p)[off(e)]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] = static_cast<float>(static_cast<const _Float16*>(p)[off(e)]);
+  }
+}
+
+template <typename F>
+__device__ __forceinline__ void scatter16(void* p, int dtype, F&& off, const float (&x)[16], int count) {
+  if (dtype == TF_FLOAT32) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (e < count) static_cast<float*>(p)[off(e)] = x[e];
+  } else if (dtype == TF_BFLOAT16) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (e < count) static_cast<uint16_t*>(p)[off(e)] = f32_to_bf16(x[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (e < count) static_cast<_Float16*>(p)[off(e)] = static_cast<_Float16>(x[e]);
+  }
+}
+
+// NT: 32-channel tiles of the state dim. RP: phase pairs per wave (8 RP >= R).
+// ROUND: some operand is 16-bit, so the rounding points are not the identity.
+template <int NT, int RP, bool ROUND, typename I>
+__global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericParams<I> P) {
   using Sm = GenericShared<NT>;
   constexpr int NS = Sm::NS, TS = Sm::TS, VS = Sm::VS, SS = Sm::SS;
   __shared__ __align__(16) Sm sh;
+  const tf_mamba_args& a = P.a;
   const int h = blockIdx.x;
   const int b = blockIdx.y;
-  const int tid = static_cast<int>(threadIdx.x);
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int c32 = lane & 31, hh = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int n_state = static_cast<int>(a.state);
   const int p_dim = static_cast<int>(a.head_dim);
   const int rot = static_cast<int>(a.rotary);
@@ -145,26 +205,24 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
   // reverse: step t < L reads and writes row L-1-t; steps >= L have no row
   const bool rev = a.reverse != 0;
   const int tlim = rev ? L : T;
-  auto row = [&](int t) -> int64_t { return rev ? L - 1 - t : t; };
+  const I roff = rev ? max(L - 1, 0) : 0;
   auto rnd = [](float x, int dtype) { return ROUND ? round_to(x, dtype) : x; };
   const bool raw = a.dt_bias != nullptr;
   const bool norm = a.q_norm != nullptr;
   const float step_bias = raw ? a.dt_bias[h] : 0.f;
 
-  const int64_t qo = b * a.q_stride[0] + qh * a.q_stride[2];
-  const int64_t ko = b * a.k_stride[0] + qh * a.k_stride[2];
-  const int64_t vo = b * a.v_stride[0] + h * a.v_stride[2];
-  const int64_t zo = b * a.z_stride[0] + h * a.z_stride[2];
-  const int64_t oo = b * a.out_stride[0] + h * a.out_stride[2];
-  const int64_t go = b * a.angles_stride[0] + h * a.angles_stride[2];
-  const int64_t ao = b * a.adt_stride[0] + h * a.adt_stride[1];
-  const int64_t dto = b * a.dt_stride[0] + h * a.dt_stride[1];
-  const int64_t tro = b * a.trap_stride[0] + h * a.trap_stride[1];
+  const I qo = b * P.q[0] - roff * P.q[1] + qh * P.q[2];
+  const I ko = b * P.k[0] - roff * P.k[1] + qh * P.k[2];
+  const I vo = b * P.v[0] - roff * P.v[1] + h * P.v[2];
+  const I zo = b * P.z[0] - roff * P.z[1] + h * P.z[2];
+  const I oo = b * P.o[0] - roff * P.o[1] + h * P.o[2];
+  const I go = b * P.g[0] - roff * P.g[1] + h * P.g[2];
+  const I ao = b * P.ad[0] + h * P.ad[1] - roff * P.ad[2];
+  const I dto = b * P.dt[0] + h * P.dt[1] - roff * P.dt[2];
+  const I tro = b * P.tr[0] + h * P.tr[1] - roff * P.tr[2];
 
   const float skip = a.d[h];
   const int nchunks = (L + kChunk - 1) / kChunk;
-  const int rrow = tid / kRowLanes, grp = tid % kRowLanes;  // rotation: row and channel group
-  const int rp = (rot + 7) / 8;                             // phase pairs per wave
   // output waves: rows 32 th .., columns 32 pt ..; state waves: tiles s, s + 4 of (n, p)
   const int PT = p_dim > 32 ? 2 : 1;
   const int th = (w & 3) >> 1, pt = w & 1;
@@ -173,60 +231,78 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
 
   // raw operands of one chunk, requested one chunk ahead
   float4 xq[NT], xk[NT], xv[2];
-  float ang[kPairsPerWave];
+  float ang[RP];
   float c_dt = 0.f, c_dn = 0.f, c_ad = 0.f, c_tr = 0.f, c_tn = 0.f;
-  auto load_chunk = [&](int c) {
+  auto load_chunk = [&](int c, int tid) {
+    const int lane = tid & 63, rrow = tid / kRowLanes, grp = tid % kRowLanes;
     const int t = c * kChunk + rrow;
-    const int64_t r = row(min(t, L - 1));
+    const I r = min(t, L - 1);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      xq[j] = load_piece(a.q, a.q_dtype, qo + r * a.q_stride[1], a.q_stride[3], 4 * grp + 32 * j, n_state, vec.q);
-      xk[j] = load_piece(a.k, a.k_dtype, ko + r * a.k_stride[1], a.k_stride[3], 4 * grp + 32 * j, n_state, vec.k);
+      xq[j] = load_piece(a.q, a.q_dtype, qo + r * P.q[1], P.q[3], 4 * grp + 32 * j, n_state, P.qvec);
+      xk[j] = load_piece(a.k, a.k_dtype, ko + r * P.k[1], P.k[3], 4 * grp + 32 * j, n_state, P.kvec);
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
-      xv[j] = load_piece(a.v, a.v_dtype, vo + r * a.v_stride[1], a.v_stride[3], 4 * grp + 32 * j, p_dim, vec.v);
+      xv[j] = load_piece(a.v, a.v_dtype, vo + r * P.v[1], P.v[3], 4 * grp + 32 * j, p_dim, P.vvec);
     const int tl = c * kChunk + lane;
-    const int64_t rl = row(min(tl, L - 1));
+    const I rl = min(tl, L - 1);
 #pragma unroll
-    for (int i = 0; i < kPairsPerWave; ++i) {
-      const int pair = w * rp + i;
-      ang[i] = i < rp && pair < rot
-                   ? load_f32(a.angles, a.angles_dtype, go + rl * a.angles_stride[1] + pair * a.angles_stride[3])
-                   : 0.f;
+    for (int i = 0; i < RP; ++i) {
+      const int pair = w * RP + i;
+      ang[i] = pair < rot ? load_f32(a.angles, a.angles_dtype, go + rl * P.g[1] + pair * P.g[3]) : 0.f;
     }
     if (w == 0) {
-      const bool valid = tl < L, next = tl + 1 < tlim;
-      c_dt = valid ? load_f32(a.dt, a.dt_dtype, dto + rl * a.dt_stride[2]) : 0.f;
-      c_dn = next ? load_f32(a.dt, a.dt_dtype, dto + row(tl + 1) * a.dt_stride[2]) : 0.f;
-      c_ad = valid ? load_f32(a.adt, a.adt_dtype, ao + rl * a.adt_stride[2]) : 0.f;
-      c_tr = valid ? load_f32(a.trap, a.trap_dtype, tro + rl * a.trap_stride[2]) : 0.f;
-      c_tn = next ? load_f32(a.trap, a.trap_dtype, tro + row(tl + 1) * a.trap_stride[2]) : 0.f;
+      // rows clamped to ones that exist, masked where used
+      const I rn = max(min(tl + 1, tlim - 1), 0);
+      c_dt = load_f32(a.dt, a.dt_dtype, dto + rl * P.dt[2]);
+      c_dn = load_f32(a.dt, a.dt_dtype, dto + rn * P.dt[2]);
+      c_ad = load_f32(a.adt, a.adt_dtype, ao + rl * P.ad[2]);
+      c_tr = load_f32(a.trap, a.trap_dtype, tro + rl * P.tr[2]);
+      c_tn = load_f32(a.trap, a.trap_dtype, tro + rn * P.tr[2]);
     }
   };
 
   f32x16 state[2] = {zero16(), zero16()};  // state waves
-  double carry[kPairsPerWave];             // phase entering the chunk, revolutions
+  double carry[RP];             // phase entering the chunk, revolutions
 #pragma unroll
-  for (int i = 0; i < kPairsPerWave; ++i) carry[i] = 0.0;
-  for (int e = tid; e < kPMax * NS; e += kThreads) sh.st[e] = 0.f;
-  if (nchunks > 0) load_chunk(0);
+  for (int i = 0; i < RP; ++i) carry[i] = 0.0;
+  for (int e = static_cast<int>(threadIdx.x); e < kPMax * NS; e += kThreads) sh.st[e] = 0.f;
+  for (int e = static_cast<int>(threadIdx.x); e < Sm::NP; e += kThreads) {
+    const bool on = e < n_state;
+    sh.qb[e] = on ? a.qb[h * n_state + e] : 0.f;
+    sh.kb[e] = on ? a.kb[h * n_state + e] : 0.f;
+    sh.qw[e] = on && norm ? a.q_norm[e] : 0.f;
+    sh.kw[e] = on && norm ? a.k_norm[e] : 0.f;
+  }
+  if (nchunks > 0) load_chunk(0, static_cast<int>(threadIdx.x));
 
   for (int c = 0; c < nchunks; ++c) {
     const int t0 = c * kChunk;
+    // lane-derived indices from a thread index the compiler cannot see through:
+    // hoisted out of the loop, the addresses they feed would live across it
+    // and spill
+    int tid = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63;
+    const int c32 = lane & 31, hh = lane >> 5;
+    const int rrow = tid / kRowLanes, grp = tid % kRowLanes;  // rotation: row and channel group
     if (w == 0) {
       const int t = t0 + lane;
       const bool valid = t < L, next = t + 1 < tlim;
       float dt = c_dt, dn = c_dn, ad = c_ad;
       if (raw) {  // controls from the raw a/ddt columns (primitives.py:209-214)
-        dt = valid ? control_step(dt, step_bias) : 0.f;
-        dn = next ? control_step(dn, step_bias) : 0.f;
-        ad = valid ? control_decay(ad, dt, a.a_floor) : 0.f;
+        dt = control_step(dt, step_bias);
+        dn = control_step(dn, step_bias);
+        ad = control_decay(ad, dt, a.a_floor);
       }
-      const float tr = sigmoid_exact(c_tr), tn = sigmoid_exact(c_tn);
+      dt = valid ? dt : 0.f;
+      dn = next ? dn : 0.f;
+      ad = valid ? ad : 0.f;
+      const float tr = sigmoid_exact(valid ? c_tr : 0.f), tn = sigmoid_exact(next ? c_tn : 0.f);
       const float gamma = dt * tr;
-      const float cs = wave_inclusive_scan(ad * kLog2e);
-      const float tot = __shfl(cs, 63, 64);
+      const float cs = wave_scan_dpp(ad * kLog2e);
+      const float tot = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cs), 63));
       sh.cs[lane] = cs;
       sh.wv[lane] = exp2f(tot - cs);
       sh.ecs[lane] = exp2f(cs);
@@ -236,26 +312,25 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
       if (lane == 0) sh.wild = 0;
     }
     // the rotary's tanh does not wait for the controls
-    double om[kPairsPerWave];
+    double om[RP];
 #pragma unroll
-    for (int i = 0; i < kPairsPerWave; ++i)
-      if (i < rp) om[i] = tanh_f64(static_cast<double>(ang[i]));
+    for (int i = 0; i < RP; ++i) om[i] = tanh_f64(static_cast<double>(ang[i]));
     __syncthreads();
     // phase in revolutions, accumulated in fp64 (mamba_fused.py:102-111): pi tanh dt
     // radians = tanh dt / 2 revolutions; rows past the length add 0
     {
       const double dt = static_cast<double>(sh.dt[lane]);
 #pragma unroll
-      for (int i = 0; i < kPairsPerWave; ++i) {
-        const int pair = w * rp + i;
-        if (i < rp && pair < rot) {
+      for (int i = 0; i < RP; ++i) {
+        const int pair = w * RP + i;
+        if (pair < rot) {
           const double inc = t0 + lane < L ? om[i] * dt * 0.5 : 0.0;
-          const double sum = wave_scan_f64(inc, lane) + carry[i];
+          const double sum = wave_scan_f64(inc) + carry[i];
           const float rev2 = static_cast<float>(2.0 * (sum - __builtin_rint(sum)));
           float si, co;
           sincospif(rev2, &si, &co);
           *reinterpret_cast<float2*>(&sh.trig[lane * TS + 2 * pair]) = make_float2(co, si);
-          const double last = __shfl(sum, 63, 64);
+          const double last = last_lane_f64(sum);
           carry[i] = last - __builtin_rint(last);
         }
       }
@@ -284,16 +359,13 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
         float q[4] = {xq[j].x, xq[j].y, xq[j].z, xq[j].w}, k[4] = {xk[j].x, xk[j].y, xk[j].z, xk[j].w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const int n = n0 + e;
-          if (n < n_state) {
-            if (norm) {
-              // rounded to the operand dtype as the norm's output is
-              q[e] = rnd(q[e] * rq * a.q_norm[n], a.q_dtype);
-              k[e] = rnd(k[e] * rk * a.k_norm[n], a.k_dtype);
-            }
-            q[e] += a.qb[h * n_state + n];
-            k[e] += a.kb[h * n_state + n];
+          if (norm) {
+            // rounded to the operand dtype as the norm's output is
+            q[e] = rnd(q[e] * rq * sh.qw[n0 + e], a.q_dtype);
+            k[e] = rnd(k[e] * rk * sh.kw[n0 + e], a.k_dtype);
           }
+          q[e] += sh.qb[n0 + e];
+          k[e] += sh.kb[n0 + e];
           dot += q[e] * k[e];  // unrotated biased vectors (:124)
         }
         float qv[4], kv[4];
@@ -327,16 +399,11 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
     const bool late = t0 + 32 >= L;  // the chunk's second half has no valid row
     const bool y_on = out_wave && !(late && th == 1);
     if (y_on) {
-      const int p = 32 * pt + c32;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int t = t0 + 32 * th + drow(e, hh);
-        zz[e] = t < L && p < p_dim
-                    ? load_f32(a.z, a.z_dtype, zo + row(t) * a.z_stride[1] + p * a.z_stride[3])
-                    : 0.f;
-      }
+      // rows and columns clamped to ones that exist; masked at the store
+      const I zc = zo + min(32 * pt + c32, p_dim - 1) * P.z[3];
+      gather16(a.z, a.z_dtype, [&](int e) -> I { return zc + min(t0 + 32 * th + drow(e, hh), L - 1) * P.z[1]; }, zz);
     }
-    if (c + 1 < nchunks) load_chunk(c + 1);
+    if (c + 1 < nchunks) load_chunk(c + 1, tid);
     __syncthreads();
     f32x16 inter = zero16();
     if (y_on) {
@@ -388,6 +455,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
       const float* y = &sh.v[4 * hh * VS + 32 * pt + c32];
       const int p = 32 * pt + c32;
       if (!sh.wild) {
+#pragma unroll 4
         for (int s = 0; s < 4 * (th + 1); ++s) {
           const float4 xa = *reinterpret_cast<const float4*>(x + 8 * s);
           const float* yr = y + 8 * s * VS;
@@ -407,14 +475,18 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
           intra[e] = sum;
         }
       }
+      float y2[16];
+      int count = 0;  // the lane's rows below the length: they come in order
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int r = 32 * th + drow(e, hh), t = t0 + r;
-        const float y2 = inter[e] * sh.ecs[r] + intra[e] + (skip + sh.qk[r]) * sh.v[r * VS + p];
-        if (t < L && p < p_dim)
-          store_f32(a.out, a.out_dtype, oo + row(t) * a.out_stride[1] + p * a.out_stride[3],
-                    y2 * (zz[e] * sigmoidf(zz[e])));
+        const int r = 32 * th + drow(e, hh);
+        count += t0 + r < L ? 1 : 0;
+        y2[e] = inter[e] * sh.ecs[r] + intra[e] + (skip + sh.qk[r]) * sh.v[r * VS + p];
+        y2[e] *= zz[e] * sigmoidf(zz[e]);
       }
+      const I oc = oo + p * P.o[3] + (t0 + 32 * th) * P.o[1];
+      if (p < p_dim)
+        scatter16(a.out, a.out_dtype, [&](int e) -> I { return oc + drow(e, hh) * P.o[1]; }, y2, count);
     } else if (w >= 4 && c + 1 < nchunks) {
       // state update S <- S 2^tot + round_k(v 2^(tot-cs))^T kr (mamba_fused.py:150-152):
       // lane = p, values = n
@@ -443,26 +515,62 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const tf_mamba_
     __syncthreads();
   }
   // rows past the valid prefix (the same rows in either direction)
-  for (int64_t e = static_cast<int64_t>(L) * p_dim + tid; e < static_cast<int64_t>(T) * p_dim; e += kThreads) {
-    const int64_t t = e / p_dim, p = e - t * p_dim;
-    store_f32(a.out, a.out_dtype, oo + t * a.out_stride[1] + p * a.out_stride[3], 0.f);
+  const I st = rev ? -P.o[1] : P.o[1];
+  const I of = b * P.o[0] + h * P.o[2];
+  for (int t = L + w; t < T; t += kThreads / 64) {
+    const int p = static_cast<int>(threadIdx.x & 63);
+    if (p < p_dim) store_f32(a.out, a.out_dtype, of + t * st + p * P.o[3], 0.f);
   }
 }
 
-template <int NT>
-int launch_tiles(const tf_mamba_args& a, const GenericVec& vec, bool round, hipStream_t stream) {
+template <typename I>
+GenericParams<I> make_generic(const tf_mamba_args& a);
+
+template <int NT, int RP, typename I>
+int launch_pairs(const tf_mamba_args& a, hipStream_t stream) {
+  const GenericParams<I> P = make_generic<I>(a);
   const dim3 grid(static_cast<uint32_t>(a.heads), static_cast<uint32_t>(a.batch));
-  if (round)
-    hipLaunchKernelGGL((mamba_generic_kernel<NT, true>), grid, dim3(kThreads), 0, stream, a, vec);
+  if (a.q_dtype != TF_FLOAT32 || a.k_dtype != TF_FLOAT32 || a.v_dtype != TF_FLOAT32)
+    hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, true, I>), grid, dim3(kThreads), 0, stream, P);
   else
-    hipLaunchKernelGGL((mamba_generic_kernel<NT, false>), grid, dim3(kThreads), 0, stream, a, vec);
+    hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, false, I>), grid, dim3(kThreads), 0, stream, P);
   return launch_status();
+}
+
+template <int NT>
+int launch_tiles(const tf_mamba_args& a, hipStream_t stream) {
+  if (!offsets_fit(a)) return launch_pairs<NT, 2 * NT, int64_t>(a, stream);
+  // a quarter of the state dim rotates in the models; a half at most
+  if (a.rotary <= 8 * NT) return launch_pairs<NT, NT, int32_t>(a, stream);
+  return launch_pairs<NT, 2 * NT, int32_t>(a, stream);
 }
 
 // Four elements at a time: whole pieces inside the row, aligned at every row.
 int vec4(const void* p, int dtype, const int64_t* st, int64_t n) {
   const int es = dtype_size(dtype);
   return n % 4 == 0 && rows_vectorisable(p, st, es, 4 * es);
+}
+
+template <typename I>
+GenericParams<I> make_generic(const tf_mamba_args& a) {
+  GenericParams<I> P;
+  P.a = a;
+  const I sign = a.reverse ? -1 : 1;
+  auto four = [&](I(&d)[4], const int64_t* s) {
+    for (int i = 0; i < 4; ++i) d[i] = static_cast<I>(s[i]);
+    d[1] *= sign;
+  };
+  auto three = [&](I(&d)[3], const int64_t* s) {
+    for (int i = 0; i < 3; ++i) d[i] = static_cast<I>(s[i]);
+    d[2] *= sign;
+  };
+  four(P.q, a.q_stride), four(P.k, a.k_stride), four(P.v, a.v_stride), four(P.z, a.z_stride);
+  four(P.g, a.angles_stride), four(P.o, a.out_stride);
+  three(P.ad, a.adt_stride), three(P.dt, a.dt_stride), three(P.tr, a.trap_stride);
+  P.qvec = vec4(a.q, a.q_dtype, a.q_stride, a.state);
+  P.kvec = vec4(a.k, a.k_dtype, a.k_stride, a.state);
+  P.vvec = vec4(a.v, a.v_dtype, a.v_stride, a.head_dim);
+  return P;
 }
 
 }  // namespace
@@ -472,13 +580,9 @@ bool generic_supported(const tf_mamba_args& a) {
 }
 
 int launch_generic(const tf_mamba_args& a, hipStream_t stream) {
-  const GenericVec vec = {vec4(a.q, a.q_dtype, a.q_stride, a.state), vec4(a.k, a.k_dtype, a.k_stride, a.state),
-                          vec4(a.v, a.v_dtype, a.v_stride, a.head_dim)};
-  const bool round = a.q_dtype != TF_FLOAT32 || a.k_dtype != TF_FLOAT32 || a.v_dtype != TF_FLOAT32;
-  if (a.state <= 32) return launch_tiles<1>(a, vec, round, stream);
-  if (a.state <= 64) return launch_tiles<2>(a, vec, round, stream);
-  if (a.state <= 96) return launch_tiles<3>(a, vec, round, stream);
-  return launch_tiles<4>(a, vec, round, stream);
+  if (a.state <= 32) return launch_tiles<1>(a, stream);
+  if (a.state <= 64) return launch_tiles<2>(a, stream);
+  return launch_tiles<4>(a, stream);
 }
 
 }  // namespace tf
