@@ -24,6 +24,11 @@ int launch_mfma(const tf_mamba_args& a, hipStream_t stream);
 // (0: one workgroup per unit).
 int64_t mfma_workspace_bytes(const tf_mamba_args& a);
 
+// N = 128, P = 64 form of the MFMA kernel (arguments mfma_supported accepts)
+// and its scratch bytes.
+int launch_wide(const tf_mamba_args& a, hipStream_t stream);
+int64_t wide_workspace_bytes(const tf_mamba_args& a);
+
 // Pipelined MFMA kernel (N = P = 64): one workgroup walks each unit, or, for
 // few long units with a workspace, each (unit, time segment).
 bool pipe_supported(const tf_mamba_args& a);

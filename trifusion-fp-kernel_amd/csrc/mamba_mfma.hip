@@ -961,6 +961,7 @@ int launch_shape(const tf_mamba_args& a, hipStream_t stream) {
 
 int64_t mfma_workspace_bytes(const tf_mamba_args& a) {
   if (!mfma_supported(a)) return 0;
+  if (a.state == 128 && a.head_dim == 64) return wide_workspace_bytes(a);
   const SegPlan plan = plan_segments(a, shape_cw(a), static_cast<int>((padded_state(a) / 32) * (a.head_dim / 32) * 256));
   return plan.G > 1 ? plan.bytes : 0;
 }
@@ -1004,10 +1005,7 @@ int launch_mfma(const tf_mamba_args& a, hipStream_t stream) {
   if (nt == 2 && pt == 1) return launch_shape<2, 1, 4>(a, stream);
   if (nt == 2 && pt == 2) return launch_shape<2, 2, 4>(a, stream);
   if (nt == 4 && pt == 1) return launch_shape<4, 1, 2>(a, stream);
-  if (nt == 4 && pt == 2) {
-    if (a.batch * a.heads > kTargetGroups) return launch_shape<4, 2, 1>(a, stream);
-    return launch_shape<4, 2, 2>(a, stream);
-  }
+  if (nt == 4 && pt == 2) return launch_wide(a, stream);
   return TF_ERR_SHAPE;
 }
 

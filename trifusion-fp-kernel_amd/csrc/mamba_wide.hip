@@ -1,0 +1,663 @@
+// Fused Mamba-3 SISO recurrence on gfx950 bf16 MFMA for N = 128, P = 64.
+//
+// Same arithmetic and bf16 rounding points as the reference kernel
+// (src/trifusion_l4/mamba_fused.py:72-152). A workgroup of four waves walks one
+// (batch, head) unit, or one time segment of it, in 64-step chunks; two
+// workgroups share a CU (77 KB of LDS and at most 256 registers each), so one's
+// vector work covers the other's latency. Per chunk, between three barriers:
+//
+//   rotation   16 rows per wave: [B/C norm,] bias, rotation, scale; values and
+//              decay-scaled values; all to LDS as bf16 rows
+//   products 1 y^T = S^T qr^T (all steps x the wave's 16 head dims), the ten
+//              lower 16x16 score tiles shared out; one wave forms the next
+//              chunk's controls
+//   products 2 scores v, skip, gate, store; state update; the next chunk's
+//              rotary phase and cos/sin table
+//
+// Wave w holds head dims 16 w .. 16 w + 15 of the fp32 state, all 128 channels,
+// as eight 16x16 MFMA tiles. Its accumulator registers, packed to bf16, are the
+// operand of the next chunk's S qr product: the state never passes through LDS.
+//
+// MFMA 16x16x32 layout (lane l, r = l & 15, g = l >> 4):
+//   A[i][k]: lane i + 16 (k / 8), element k % 8; B[k][j]: lane j + 16 (k / 8)
+//   D[i][j]: lane j + 16 (i / 4), element i % 4
+// Contraction slots are permuted the same way on both sides: slot j of k-step s
+// holds index 32 s + 16 (j / 4) + 4 g + j % 4, which is where a pair of D tiles
+// holds its rows.
+//
+// Chunk-parallel form (few long units): summaries of every segment but the last
+// (this kernel, MODE 1: from zero state and phase, only keys and values), a scan
+// that turns each summary into the state entering the next segment, and the
+// seeded walks. A summary is formed in its segment's own phase frame; the scan
+// turns it by the phase entering the segment (mamba_pipe.hip describes why that
+// is the same state).
+#include <algorithm>
+
+#include "mamba_walk.h"
+
+namespace tf {
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+// 16 bytes of a row whose rows are 8-byte aligned
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
+
+constexpr int kWideThreads = 256;
+constexpr int kRecF4 = 2048;  // float4 per state record: [tile][thread]
+
+__device__ __forceinline__ f32x4 mfma16(const u32x4& x, const u32x4& y, const f32x4& acc) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, y), acc, 0,
+                                                 0, 0);
+}
+
+// Rows t0 .. t0 + 15 of a [64][64] row buffer as an operand of k-step s (columns 32 s ..).
+__device__ __forceinline__ u32x4 row16(const uint16_t* buf, int t0, int s, int r, int g) {
+  const u32x2 lo = rb_read(buf, t0 + r, 8 * s + g), hi = rb_read(buf, t0 + r, 8 * s + 4 + g);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// Columns 4 u0 .. 4 u0 + 15 of a [64][64] row buffer as an operand of k-step s
+// (rows 32 s ..): in each 16-lane group, source lane 4 k + c reads row k, unit c
+// of a 4 x 4 block, and output lane j receives column j of the four rows.
+template <bool BOTH>
+__device__ __forceinline__ u32x4 col16(const uint16_t* buf, int u0, int s, int r, int g) {
+  const int row = 32 * s + 4 * g + (r >> 2), u = u0 + (r & 3);
+  const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(buf + rb_off(row, u))));
+  if constexpr (!BOTH) return u32x4{lo[0], lo[1], 0u, 0u};
+  const u32x2 hi =
+      __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(buf + rb_off(row + 16, u))));
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// RT: rotary pairs the cos/sin table holds (R <= RT).
+template <int RT>
+struct WideSmem {
+  static constexpr int TS = 2 * RT + 2;  // floats per table row
+  uint16_t qr[2][64 * 64];  // bf16(rot(q + qb)), channels 0-63 and 64-127
+  uint16_t kr[2][64 * 64];  // bf16(rot(k + kb) * s)
+  uint16_t v[64 * 64];      // v (0 past the valid length)
+  uint16_t vs[64 * 64];     // bf16(v * 2^(tot - cs))
+  uint16_t sc[64 * 64];     // bf16 scores [t][u]
+  float trig[64 * TS];      // [row][pair] (cos, sin)
+  float qw[128], kw[128];   // fused B/C norm weights
+  float qb[128], kb[128];   // biases
+  // per-row controls of chunk c (c mod 2)
+  float dt[2][64], scl[2][64], cs[2][64], wv[2][64], gam[2][64];
+  float tot[2];
+  float skip[64];  // (q + qb).(k + kb) of each row
+};
+
+// Element i of a control, trapezoid or angle tensor. IN: 0 all three fp32, 1 all
+// bf16, 2 as the flag says.
+template <int IN>
+__device__ __forceinline__ float load_in(const void* base, int bf16, int i) {
+  if constexpr (IN == 2)
+    return ctl_value(base, bf16, i);
+  else
+    return load_elem<IN == 1>(base, i);
+}
+
+// Raw 16-byte pieces of one row: channels 8 ng .. and 64 + 8 ng .. of q and k,
+// head dims 8 ng .. of v.
+struct WideRow {
+  u32x4 q[2], k[2], v;
+};
+
+// Fused B/C RMSNorm (mamba.py:56-57, kernels/__init__.py:10-12) of a row of 128
+// channels, 16 in each of 8 neighbouring lanes: x -> bf16(x rsqrt(mean + eps) w).
+__device__ __forceinline__ void norm_row16(u32x4 (&x)[2], const float* w, int ng, float eps) {
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      ss = __builtin_fmaf(lo_f(x[i][j]), lo_f(x[i][j]), ss);
+      ss = __builtin_fmaf(hi_f(x[i][j]), hi_f(x[i][j]), ss);
+    }
+  const float r = rsqrtf(group8_sum(ss) / 128.f + eps);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float4 a = *reinterpret_cast<const float4*>(w + 64 * i + 8 * ng);
+    const float4 b = *reinterpret_cast<const float4*>(w + 64 * i + 8 * ng + 4);
+    const float ww[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[i][j] = pack2(lo_f(x[i][j]) * r * ww[2 * j], hi_f(x[i][j]) * r * ww[2 * j + 1]);
+  }
+}
+
+// MODE 0: outputs of the unit's (or, P.G > 1, the segment's) chunks. MODE 1: the
+// segment's state from zero, its log2 decay and phase sums.
+template <int RT, int IN, int MODE>
+__global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_kernel(const MfmaParams P) {
+  using Sm = WideSmem<RT>;
+  constexpr int TS = Sm::TS;
+  constexpr int PI = RT / 32;  // phase pairs per lane
+  __shared__ __align__(16) Sm sh;
+  const PipeItem it = pipe_item(P);
+  const int seg = it.seg, h = it.h, b = it.b;
+  if (MODE == 1 && seg == P.G - 1) return;  // no walk starts from the last segment's state
+  const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  // lane-derived indices, rebuilt every chunk from an index the compiler cannot
+  // see through: hoisted out of the walk, the LDS addresses they feed would
+  // hold a register each and spill
+  int lane, r16, g, ng, row0, pi, sg;
+  auto lane_indices = [&]() {
+    lane = static_cast<int>(threadIdx.x & 63);
+    asm volatile("" : "+v"(lane));
+    r16 = lane & 15, g = lane >> 4;
+    // rotation: rows 16 w + 8 i + row8 (i = 0, 1), eight lanes per row
+    ng = lane & 7, row0 = 16 * w + row8_of_lane(lane);
+    // phase: lane = (pair of eight, segment of eight rows), pairs 32 i + 8 w + pi
+    pi = lane >> 3, sg = lane & 7;
+  };
+  lane_indices();
+  const int T = P.T, R = P.R;
+  int L = T;
+  if (P.lengths != nullptr) {
+    const int64_t l = P.lengths[b];
+    L = l < 0 ? 0 : (l > T ? T : static_cast<int>(l));
+  }
+  const int nvalid = (L + kChunk - 1) / kChunk;
+  const int c0 = min(seg_start(P, seg), nvalid);
+  const int c1 = min(seg_start(P, seg + 1), nvalid);
+
+  if (c1 > c0) {
+    const int tlim = P.rev ? L : T;
+    const int roff = P.rev ? max(L - 1, 0) : 0;
+    const int qh = h / P.group;
+    const uint16_t* qbase = P.q + b * P.q_sb + qh * P.q_sh - roff * P.q_st;
+    const uint16_t* kbase = P.k + b * P.k_sb + qh * P.k_sh - roff * P.k_st;
+    const uint16_t* vbase = P.v + b * P.v_sb + h * P.v_sh - roff * P.v_st;
+    const uint16_t* zbase = P.z + b * P.z_sb + h * P.z_sh - roff * P.z_st;
+    const int dto = b * P.d_sb + h * P.d_sh - roff * P.d_st;
+    const int ado = b * P.a_sb + h * P.a_sh - roff * P.a_st;
+    const int trb = b * P.r_sb + h * P.r_sh - roff * P.r_st;
+    const int gbase = b * P.g_sb + h * P.g_sh - roff * P.g_st;
+    const int obase = b * P.o_sb + h * P.o_sh - roff * P.o_st;
+    const float step_bias = P.ctl_raw ? P.dt_bias[h] : 0.f;
+    const float skip_d = MODE == 0 ? P.d[h] : 0.f;
+    const int ang16 = P.angles_dtype == TF_BFLOAT16;
+
+    auto load_rows = [&](int c, WideRow (&x)[2]) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int t = min(c * kChunk + row0 + 8 * i, L - 1);
+        const uint16_t* kp = kbase + t * P.k_st + 8 * ng;
+        x[i].k[0] = *reinterpret_cast<const u32x4_a8*>(kp);
+        x[i].k[1] = *reinterpret_cast<const u32x4_a8*>(kp + 64);
+        x[i].v = *reinterpret_cast<const u32x4_a8*>(vbase + t * P.v_st + 8 * ng);
+        if constexpr (MODE == 0) {
+          const uint16_t* qp = qbase + t * P.q_st + 8 * ng;
+          x[i].q[0] = *reinterpret_cast<const u32x4_a8*>(qp);
+          x[i].q[1] = *reinterpret_cast<const u32x4_a8*>(qp + 64);
+        }
+      }
+    };
+    // controls: wave 3, lane = row; rows clamped to ones that exist
+    auto load_ctl = [&](int c) {
+      const int tc = min(c * kChunk + lane, L - 1), tn = min(c * kChunk + lane + 1, tlim - 1);
+      PipeCtl x;
+      x.dt = load_in<IN>(P.dt, P.ctl_bf16, dto + tc * P.d_st);
+      x.dn = load_in<IN>(P.dt, P.ctl_bf16, dto + tn * P.d_st);
+      x.adt = load_in<IN>(P.adt, P.ctl_bf16, ado + tc * P.a_st);
+      x.tr = load_in<IN>(P.trap, P.trap_bf16, trb + tc * P.r_st);
+      x.tn = load_in<IN>(P.trap, P.trap_bf16, trb + tn * P.r_st);
+      return x;
+    };
+    float seg_log2 = 0.f;
+    auto controls = [&](const PipeCtl& raw, int c) {
+      const int t = c * kChunk + lane, cb = c & 1;
+      const RowControls rc = row_controls(P, raw, t < L, t + 1 < tlim, step_bias);
+      sh.dt[cb][lane] = rc.dt;
+      sh.scl[cb][lane] = rc.sc;
+      sh.cs[cb][lane] = rc.cs;
+      sh.wv[cb][lane] = rc.wv;
+      sh.gam[cb][lane] = rc.gam;
+      if (lane == 0) sh.tot[cb] = rc.tot;
+    };
+    auto load_angles = [&](int c, float (&th)[PI][8]) {
+#pragma unroll
+      for (int i = 0; i < PI; ++i) {
+        const int pair = 32 * i + 8 * w + pi;
+        const int col = gbase + (pair < R ? pair : 0) * P.g_sr;
+        if (32 * i + 8 * w < R) {  // wave-uniform
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            th[i][j] = load_in<IN>(P.angles, ang16, col + min(c * kChunk + 8 * sg + j, L - 1) * P.g_st);
+        }
+      }
+    };
+    uint32_t carry[PI];  // phase entering the chunk, 2^-32 revolutions
+#pragma unroll
+    for (int i = 0; i < PI; ++i) {
+      carry[i] = 0;
+      if (MODE == 0 && P.G > 1) {
+        // the wrapping sum of the preceding segments' phase sums
+        const int pair = 32 * i + 8 * w + pi;
+        uint32_t part = 0;
+        if (pair < R)
+          for (int s = sg; s < seg; s += 8) part += P.phase_fx[(static_cast<size_t>(it.unit) * P.G + s) * RT + pair];
+        const uint32_t incl = group_scan_dpp<8>(part, lane);
+        carry[i] = __shfl(incl, lane | 7, 64);
+      }
+    }
+    auto phase = [&](const float (&th)[PI][8], int c) {
+      const float* dts = &sh.dt[c & 1][8 * sg];
+      const float4 da = *reinterpret_cast<const float4*>(dts), db = *reinterpret_cast<const float4*>(dts + 4);
+      const float dt[8] = {da.x, da.y, da.z, da.w, db.x, db.y, db.z, db.w};
+#pragma unroll
+      for (int i = 0; i < PI; ++i) {
+        if (32 * i + 8 * w < R) {
+          uint32_t loc[8], run = 0;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            run += phase_inc(th[i][j], dt[j]);
+            loc[j] = run;
+          }
+          const uint32_t incl = group_scan_dpp<8>(run, lane);
+          const uint32_t base = carry[i] + (incl - run);
+          const int pair = 32 * i + 8 * w + pi;
+          if (pair < R) {
+            float* tg = &sh.trig[8 * sg * TS + 2 * pair];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              float2 x = phase_trig(base + loc[j]);
+              // an angle that is not a number makes its row (and with it every
+              // later one) not a number; fixed point alone would lose it
+              x.x = th[i][j] == th[i][j] ? x.x : th[i][j];
+              *reinterpret_cast<float2*>(tg + j * TS) = x;
+            }
+          }
+          carry[i] += __shfl(incl, lane | 7, 64);
+        }
+      }
+    };
+    // norm, bias, rotation, scale and rounding of the lane's row pieces
+    // (mamba_fused.py:112-135, 151; mamba.py:56-57)
+    auto rotate = [&](WideRow (&x)[2], int c) {
+      const int cb = c & 1;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = row0 + 8 * i;
+        const bool valid = c * kChunk + row < L;
+        const float scl = sh.scl[cb][row], wvt = sh.wv[cb][row];
+        if (P.qk_norm) {
+          norm_row16(x[i].k, sh.kw, ng, P.norm_eps);
+          if constexpr (MODE == 0) norm_row16(x[i].q, sh.qw, ng, P.norm_eps);
+        }
+        float part = 0.f;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          u32x4 qo, ko;
+          float kbv[8], qbv[8];
+#pragma unroll
+          for (int j = 0; j < 8; j += 4) {
+            const float4 kb4 = *reinterpret_cast<const float4*>(&sh.kb[64 * p + 8 * ng + j]);
+            kbv[j] = kb4.x, kbv[j + 1] = kb4.y, kbv[j + 2] = kb4.z, kbv[j + 3] = kb4.w;
+            if constexpr (MODE == 0) {
+              const float4 qb4 = *reinterpret_cast<const float4*>(&sh.qb[64 * p + 8 * ng + j]);
+              qbv[j] = qb4.x, qbv[j + 1] = qb4.y, qbv[j + 2] = qb4.z, qbv[j + 3] = qb4.w;
+            }
+          }
+          if (32 * p < R) {  // wave-uniform: the piece holds rotary pairs
+            const float2* tg = reinterpret_cast<const float2*>(&sh.trig[row * TS + 64 * p + 8 * ng]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float2 cs = tg[j];
+              // pairs >= R turn by the identity
+              const bool on = 32 * p + 4 * ng + j < R;
+              const float cv = on ? cs.x : 1.f, sv = on ? cs.y : 0.f;
+              const float k0 = lo_f(x[i].k[p][j]) + kbv[2 * j], k1 = hi_f(x[i].k[p][j]) + kbv[2 * j + 1];
+              ko[j] = key_pair(k0, k1, cv, sv, scl);
+              if constexpr (MODE == 0) {
+                const float q0 = lo_f(x[i].q[p][j]) + qbv[2 * j], q1 = hi_f(x[i].q[p][j]) + qbv[2 * j + 1];
+                part += q0 * k0 + q1 * k1;
+                qo[j] = pack2(q0 * cv - q1 * sv, q0 * sv + q1 * cv);
+              }
+            }
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float k0 = lo_f(x[i].k[p][j]) + kbv[2 * j], k1 = hi_f(x[i].k[p][j]) + kbv[2 * j + 1];
+              ko[j] = pack2(k0 * scl, k1 * scl);
+              if constexpr (MODE == 0) {
+                const float q0 = lo_f(x[i].q[p][j]) + qbv[2 * j], q1 = hi_f(x[i].q[p][j]) + qbv[2 * j + 1];
+                part += q0 * k0 + q1 * k1;
+                qo[j] = pack2(q0, q1);
+              }
+            }
+          }
+          rb_write16(sh.kr[p], row, 2 * ng, ko);
+          if constexpr (MODE == 0) rb_write16(sh.qr[p], row, 2 * ng, qo);
+        }
+        u32x4 vo, vso;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          vo[j] = valid ? x[i].v[j] : 0u;
+          vso[j] = scaled_pair(vo[j], wvt);
+        }
+        rb_write16(sh.vs, row, 2 * ng, vso);
+        if constexpr (MODE == 0) {
+          rb_write16(sh.v, row, 2 * ng, vo);
+          part = group8_sum(part);
+          if (ng == 0) sh.skip[row] = part;
+        }
+      }
+    };
+
+    // the start's loads, then chunk c0's controls and phase
+    WideRow rows[2];
+    PipeCtl ctl = {};
+    float th[PI][8];
+    if (w == 3) ctl = load_ctl(c0);
+    load_angles(c0, th);
+    load_rows(c0, rows);
+    f32x4 S[8];  // state tiles [2 s + a]: channels 32 s + 16 a + 4 g + e, head dim 16 w + r16
+#pragma unroll
+    for (int j = 0; j < 8; ++j) S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bool have_state = false;
+    if (MODE == 0 && seg > 0) {
+      have_state = true;
+      const float4* rec = P.seg_state + (static_cast<size_t>(it.unit) * (P.G - 1) + seg - 1) * kRecF4 + threadIdx.x;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) S[j] = __builtin_bit_cast(f32x4, rec[j * kWideThreads]);
+    }
+    if (threadIdx.x < 128) {
+      sh.kb[threadIdx.x] = P.kb[h * 128 + threadIdx.x];
+      if (MODE == 0) sh.qb[threadIdx.x] = P.qb[h * 128 + threadIdx.x];
+      if (P.qk_norm) {
+        sh.kw[threadIdx.x] = P.kn_w[threadIdx.x];
+        if (MODE == 0) sh.qw[threadIdx.x] = P.qn_w[threadIdx.x];
+      }
+    }
+    if (w == 3) controls(ctl, c0);
+    lds_barrier();
+    phase(th, c0);
+    if (c0 + 1 < c1) {
+      if (w == 3) ctl = load_ctl(c0 + 1);
+      load_angles(c0 + 1, th);
+    }
+    lds_barrier();
+
+    for (int c = c0; c < c1; ++c) {
+      lane_indices();
+      const int cb = c & 1;
+      const int nrows = L - c * kChunk;  // valid rows of the chunk (may exceed 64)
+      const bool more = c + 1 < c1;
+      // a wave whose rows all lie past the length has none to rotate
+      if (16 * w < nrows) rotate(rows, c);
+      u32x2 zr[4];
+      if constexpr (MODE == 0) {
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+          const int t = min(c * kChunk + 16 * tt + r16, L - 1);
+          zr[tt] = *reinterpret_cast<const u32x2*>(zbase + t * P.z_st + 16 * w + 4 * g);
+        }
+      }
+      if (more) load_rows(c + 1, rows);
+      lds_barrier();
+
+      f32x4 y[4];
+      if constexpr (MODE == 0) {
+        u32x4 sp[4], kop[4];
+        if (have_state) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            sp[s] = u32x4{pack2(S[2 * s][0], S[2 * s][1]), pack2(S[2 * s][2], S[2 * s][3]),
+                          pack2(S[2 * s + 1][0], S[2 * s + 1][1]), pack2(S[2 * s + 1][2], S[2 * s + 1][3])};
+        }
+        if (16 * w < nrows) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) kop[s] = row16(sh.kr[s >> 1], 16 * w, s & 1, r16, g);
+        }
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+          y[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (16 * tt < nrows) {
+            u32x4 qop[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) qop[s] = row16(sh.qr[s >> 1], 16 * tt, s & 1, r16, g);
+            if (have_state) {
+#pragma unroll
+              for (int s = 0; s < 4; ++s) y[tt] = mfma16(sp[s], qop[s], y[tt]);
+            }
+            // scores^T tile (u, tt): kr_u . qr_t times 2^min(cs_t - cs_u, 0), strictly
+            // causal (mamba_fused.py:144-146). Tile u = w, except that wave 3 takes
+            // (0, 3) from wave 0.
+            auto score = [&](const u32x4 (&ko)[4], int u) {
+              f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int s = 0; s < 4; ++s) a = mfma16(ko[s], qop[s], a);
+              const float cst = sh.cs[cb][16 * tt + r16];
+              const float4 cu = *reinterpret_cast<const float4*>(&sh.cs[cb][16 * u + 4 * g]);
+              const float csu[4] = {cu.x, cu.y, cu.z, cu.w};
+              float x[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                // masked elements may overflow here; the select drops them
+                const float v = a[e] * fast_exp2(fminf(cst - csu[e], 0.f));
+                x[e] = (u < tt || r16 > 4 * g + e) ? v : 0.f;
+              }
+              *reinterpret_cast<u32x2*>(sh.sc + rb_off(16 * tt + r16, 4 * u + g)) =
+                  u32x2{pack2(x[0], x[1]), pack2(x[2], x[3])};
+            };
+            if (w <= tt && !(w == 0 && tt == 3)) score(kop, w);
+            if (w == 3 && tt == 3) {
+              u32x4 k0[4];
+#pragma unroll
+              for (int s = 0; s < 4; ++s) k0[s] = row16(sh.kr[s >> 1], 0, s & 1, r16, g);
+              score(k0, 0);
+            }
+          }
+        }
+      }
+      if (more && w == 3) controls(ctl, c + 1);
+      lds_barrier();
+
+      if constexpr (MODE == 0) {
+        u32x4 va[2];
+        va[0] = col16<true>(sh.v, 4 * w, 0, r16, g);
+        va[1] = col16<true>(sh.v, 4 * w, 1, r16, g);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+          if (16 * tt < nrows) {
+            const int row = 16 * tt + r16;
+            const float decay = fast_exp2(sh.cs[cb][row]);
+            const float coef = skip_d + sh.gam[cb][row] * sh.skip[row];
+            const u32x2 vv = rb_read(sh.v, row, 4 * w + g);
+            const float vf[4] = {lo_f(vv[0]), hi_f(vv[0]), lo_f(vv[1]), hi_f(vv[1])};
+            f32x4 a;
+            // (D + gamma (q + qb).(k + kb)) v + 2^cs qr . bf16(S)^T (mamba_fused.py:124, 143, 147)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] = coef * vf[e] + y[tt][e] * decay;
+            // scores . v: steps u of the score tiles (0 .. tt, tt) alone; the slots
+            // past them are 0 on both sides
+#pragma unroll
+            for (int s = 0; s <= tt / 2; ++s) {
+              if (2 * s + 1 <= tt) {
+                a = mfma16(va[s], row16(sh.sc, 16 * tt, s, r16, g), a);
+              } else {
+                const u32x2 lo = rb_read(sh.sc, row, 8 * s + g);
+                a = mfma16(u32x4{va[s][0], va[s][1], 0u, 0u}, u32x4{lo[0], lo[1], 0u, 0u}, a);
+              }
+            }
+            const int t = c * kChunk + row;
+            const float zf[4] = {lo_f(zr[tt][0]), hi_f(zr[tt][0]), lo_f(zr[tt][1]), hi_f(zr[tt][1])};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a[e] *= zf[e] * sigmoid_fast(zf[e]);
+            if (t < L) {
+              const int off = obase + t * P.o_st + 16 * w + 4 * g;
+              if (P.out_f32)
+                *reinterpret_cast<float4*>(static_cast<float*>(P.out) + off) = make_float4(a[0], a[1], a[2], a[3]);
+              else
+                *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(P.out) + off) =
+                    u32x2{pack2(a[0], a[1]), pack2(a[2], a[3])};
+            }
+          }
+        }
+      }
+      // S <- S 2^tot + kr^T . vs (mamba_fused.py:150-152); nothing follows the
+      // last valid chunk
+      if (c + 1 < nvalid) {
+        const float tot = sh.tot[cb];
+        const float dec = fast_exp2(tot);
+        seg_log2 += tot;
+        const u32x4 vb0 = col16<true>(sh.vs, 4 * w, 0, r16, g), vb1 = col16<true>(sh.vs, 4 * w, 1, r16, g);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint16_t* buf = sh.kr[j >> 2];
+          const int u0 = 4 * (j & 3);
+          f32x4 a = S[j];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) a[e] *= dec;
+          a = mfma16(col16<true>(buf, u0, 0, r16, g), vb0, a);
+          S[j] = mfma16(col16<true>(buf, u0, 1, r16, g), vb1, a);
+        }
+        have_state = true;
+      }
+      if (more) {
+        phase(th, c + 1);
+        if (c + 2 < c1) {
+          if (w == 3) ctl = load_ctl(c + 2);
+          load_angles(c + 2, th);
+        }
+      }
+      lds_barrier();
+    }
+    if constexpr (MODE == 1) {
+      float4* rec = P.seg_state + (static_cast<size_t>(it.unit) * (P.G - 1) + seg) * kRecF4 + threadIdx.x;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rec[j * kWideThreads] = __builtin_bit_cast(float4, S[j]);
+      if (threadIdx.x == 0) P.seg_decay[it.rec] = seg_log2;
+#pragma unroll
+      for (int i = 0; i < PI; ++i)
+        if (sg == 0) P.phase_fx[static_cast<size_t>(it.rec) * RT + 32 * i + 8 * w + pi] = carry[i];
+    }
+  }
+  if constexpr (MODE == 0) {
+    // the segment's rows in [L, T): the same rows in either direction
+    const int o_st = P.rev ? -P.o_st : P.o_st;
+    const int obase = b * P.o_sb + h * P.o_sh;
+    const int row_end = min(seg_start(P, seg + 1) * kChunk, T);
+    for (int e = max(seg_start(P, seg) * kChunk, L) * 16 + static_cast<int>(threadIdx.x); e < row_end * 16;
+         e += kWideThreads) {
+      const int off = obase + (e >> 4) * o_st + 4 * (e & 15);
+      if (P.out_f32)
+        *reinterpret_cast<float4*>(static_cast<float*>(P.out) + off) = make_float4(0.f, 0.f, 0.f, 0.f);
+      else
+        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(P.out) + off) = u32x2{0u, 0u};
+    }
+  }
+}
+
+// Replaces each unit's summaries by the states entering the next segments:
+// S_1 = d_0, S_{g+1} = S_g 2^dec_g + turn_g(d_g), where turn_g rotates the rotary
+// row pairs by the phase entering segment g. Workgroup (unit, slice of 64 float4).
+template <int RT>
+__global__ __launch_bounds__(64) void wide_scan_kernel(const MfmaParams P) {
+  constexpr int kSlices = kRecF4 / 64;
+  constexpr int kBatch = 8;
+  const int unit = blockIdx.x / kSlices;
+  const int f = (blockIdx.x - unit * kSlices) * 64 + threadIdx.x;
+  const int G = P.G, R = P.R;
+  // float4 f: tile f / 256, lane f % 64: channels 16 tile + 4 g + e, rotary pairs rp, rp + 1
+  const int rp = 8 * (f >> 8) + 2 * ((f & 63) >> 4);
+  float4* st = P.seg_state + static_cast<size_t>(unit) * (G - 1) * kRecF4 + f;
+  const float* dec = P.seg_decay + static_cast<size_t>(unit) * G;
+  const uint32_t* phs = P.phase_fx + static_cast<size_t>(unit) * G * RT + (rp < RT ? rp : 0);
+  const bool turn = rp < R;
+  float4 run = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint2 ph = make_uint2(0u, 0u);
+  for (int g0 = 0; g0 < G - 1; g0 += kBatch) {
+    float4 d[kBatch];
+    float m[kBatch];
+    uint2 s[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (g0 + j < G - 1) {
+        d[j] = st[static_cast<size_t>(g0 + j) * kRecF4];
+        m[j] = fast_exp2(dec[g0 + j]);
+        if (turn) s[j] = *reinterpret_cast<const uint2*>(phs + (g0 + j) * RT);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (g0 + j < G - 1) {
+        if (turn) {
+          if (g0 + j > 0) d[j] = turn_rows(d[j], ph, rp, R);
+          ph = make_uint2(ph.x + s[j].x, ph.y + s[j].y);
+        }
+        run = state_step(run, m[j], d[j]);
+        st[static_cast<size_t>(g0 + j) * kRecF4] = run;
+      }
+    }
+  }
+}
+
+// Chunk-parallel plan: segments of at least kMinChunks chunks, about kGroups
+// workgroups, and records that fit the library's static scratch.
+constexpr int64_t kGroups = 512, kMinChunks = 2, kMaxUnits = 128, kMaxRecords = 480;
+
+struct WidePlan {
+  int G = 1;
+  int64_t phase_off = 0, decay_off = 0, bytes = 0;
+};
+
+int table_pairs(const tf_mamba_args& a) { return a.rotary <= 32 ? 32 : 64; }
+
+WidePlan wide_plan(const tf_mamba_args& a) {
+  WidePlan p;
+  const int64_t units = a.batch * a.heads;
+  const int64_t chunks = (a.time + kChunk - 1) / kChunk;
+  if (units <= 0 || units > kMaxUnits) return p;
+  const int64_t g = std::min({kGroups / units, chunks / kMinChunks, kMaxRecords / units + 1});
+  if (g < 2) return p;
+  p.G = static_cast<int>(g);
+  auto up = [](int64_t x) { return (x + 255) & ~int64_t(255); };
+  p.phase_off = up(units * (g - 1) * kRecF4 * 16);
+  p.decay_off = p.phase_off + up(units * g * table_pairs(a) * 4);
+  p.bytes = p.decay_off + up(units * g * 4);
+  return p;
+}
+
+template <int RT, int IN>
+int launch_wide_kernel(const MfmaParams& P, hipStream_t stream) {
+  const dim3 grid(static_cast<uint32_t>(P.units) * P.G), block(kWideThreads);
+  if (P.G > 1) {
+    hipLaunchKernelGGL((mamba_wide_kernel<RT, IN, 1>), grid, block, 0, stream, P);
+    if (const int rc = launch_status()) return rc;
+    hipLaunchKernelGGL((wide_scan_kernel<RT>), dim3(static_cast<uint32_t>(P.units) * (kRecF4 / 64)), dim3(64), 0,
+                       stream, P);
+    if (const int rc = launch_status()) return rc;
+  }
+  hipLaunchKernelGGL((mamba_wide_kernel<RT, IN, 0>), grid, block, 0, stream, P);
+  return launch_status();
+}
+
+}  // namespace
+
+int64_t wide_workspace_bytes(const tf_mamba_args& a) {
+  const WidePlan plan = wide_plan(a);
+  return plan.G > 1 ? plan.bytes : 0;
+}
+
+int launch_wide(const tf_mamba_args& a, hipStream_t stream) {
+  MfmaParams P = make_params(a);
+  const WidePlan plan = wide_plan(a);
+  if (plan.G > 1 && a.workspace != nullptr && aligned(a.workspace, 256) && a.workspace_bytes >= plan.bytes) {
+    char* ws = static_cast<char*>(a.workspace);
+    P.G = plan.G;
+    P.seg_state = reinterpret_cast<float4*>(ws);
+    P.phase_fx = reinterpret_cast<uint32_t*>(ws + plan.phase_off);
+    P.seg_decay = reinterpret_cast<float*>(ws + plan.decay_off);
+  }
+  const int64_t items = static_cast<int64_t>(P.units) * P.G;
+  P.xcd_per = (items % 8 == 0 && items >= 64) ? static_cast<int>(items / 8) : 0;
+  const bool ang16 = P.angles_dtype == TF_BFLOAT16;
+  if (a.rotary > 32) return launch_wide_kernel<64, 2>(P, stream);
+  if (!P.ctl_bf16 && !P.trap_bf16 && !ang16) return launch_wide_kernel<32, 0>(P, stream);
+  if (P.ctl_bf16 && P.trap_bf16 && ang16) return launch_wide_kernel<32, 1>(P, stream);
+  return launch_wide_kernel<32, 2>(P, stream);
+}
+
+}  // namespace tf
