@@ -75,7 +75,7 @@ struct WideSmem {
   static constexpr int TS = 2 * RT + 2;  // floats per table row
   uint16_t qr[2][64 * 64];  // bf16(rot(q + qb)), channels 0-63 and 64-127
   uint16_t kr[2][64 * 64];  // bf16(rot(k + kb) * s)
-  uint16_t v[64 * 64];      // v (0 past the valid length)
+  uint16_t v[64 * 64];      // v
   uint16_t vs[64 * 64];     // bf16(v * 2^(tot - cs))
   uint16_t sc[64 * 64];     // bf16 scores [t][u]
   float trig[64 * TS];      // [row][pair] (cos, sin)
@@ -103,18 +103,22 @@ struct WideRow {
   u32x4 q[2], k[2], v;
 };
 
+// acc + the squares of a bf16 pair, summed in fp32 (v_dot2_f32_bf16).
+__device__ __forceinline__ float square_sum(uint32_t x, float acc) {
+  const bf16x2 v = __builtin_bit_cast(bf16x2, x);
+  return __builtin_amdgcn_fdot2_f32_bf16(v, v, acc, false);
+}
+
 // Fused B/C RMSNorm (mamba.py:56-57, kernels/__init__.py:10-12) of a row of 128
 // channels, 16 in each of 8 neighbouring lanes: x -> bf16(x rsqrt(mean + eps) w).
 __device__ __forceinline__ void norm_row16(u32x4 (&x)[2], const float* w, int ng, float eps) {
-  float ss = 0.f;
+  float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      ss = __builtin_fmaf(lo_f(x[i][j]), lo_f(x[i][j]), ss);
-      ss = __builtin_fmaf(hi_f(x[i][j]), hi_f(x[i][j]), ss);
-    }
-  const float r = rsqrtf(group8_sum(ss) / 128.f + eps);
+  for (int j = 0; j < 4; ++j) {
+    s0 = square_sum(x[0][j], s0);
+    s1 = square_sum(x[1][j], s1);
+  }
+  const float r = rsqrtf(group8_sum(s0 + s1) / 128.f + eps);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const float4 a = *reinterpret_cast<const float4*>(w + 64 * i + 8 * ng);
@@ -279,7 +283,7 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int row = row0 + 8 * i;
-        const bool valid = c * kChunk + row < L;
+        // a row past the length repeats the last one with a key scale of 0
         const float scl = sh.scl[cb][row], wvt = sh.wv[cb][row];
         if (P.qk_norm) {
           norm_row16(x[i].k, sh.kw, ng, P.norm_eps);
@@ -304,9 +308,7 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               const float2 cs = tg[j];
-              // pairs >= R turn by the identity
-              const bool on = 32 * p + 4 * ng + j < R;
-              const float cv = on ? cs.x : 1.f, sv = on ? cs.y : 0.f;
+              const float cv = cs.x, sv = cs.y;  // the identity for pairs >= R
               const float k0 = lo_f(x[i].k[p][j]) + kbv[2 * j], k1 = hi_f(x[i].k[p][j]) + kbv[2 * j + 1];
               ko[j] = key_pair(k0, k1, cv, sv, scl);
               if constexpr (MODE == 0) {
@@ -333,7 +335,7 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
         u32x4 vo, vso;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          vo[j] = valid ? x[i].v[j] : 0u;
+          vo[j] = x[i].v[j];
           vso[j] = scaled_pair(vo[j], wvt);
         }
         rb_write16(sh.vs, row, 2 * ng, vso);
@@ -355,13 +357,14 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
     f32x4 S[8];  // state tiles [2 s + a]: channels 32 s + 16 a + 4 g + e, head dim 16 w + r16
 #pragma unroll
     for (int j = 0; j < 8; ++j) S[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bool have_state = false;
     if (MODE == 0 && seg > 0) {
-      have_state = true;
       const float4* rec = P.seg_state + (static_cast<size_t>(it.unit) * (P.G - 1) + seg - 1) * kRecF4 + threadIdx.x;
 #pragma unroll
       for (int j = 0; j < 8; ++j) S[j] = __builtin_bit_cast(f32x4, rec[j * kWideThreads]);
     }
+    // pairs that do not rotate, up to the end of the last rotating piece
+    for (int e = 64 * R + static_cast<int>(threadIdx.x); e < 64 * ((R + 31) & ~31); e += kWideThreads)
+      *reinterpret_cast<float2*>(&sh.trig[(e & 63) * TS + 2 * (e >> 6)]) = make_float2(1.f, 0.f);
     if (threadIdx.x < 128) {
       sh.kb[threadIdx.x] = P.kb[h * 128 + threadIdx.x];
       if (MODE == 0) sh.qb[threadIdx.x] = P.qb[h * 128 + threadIdx.x];
@@ -400,13 +403,11 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
       f32x4 y[4];
       if constexpr (MODE == 0) {
         u32x4 sp[4], kop[4];
-        if (have_state) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
-            sp[s] = u32x4{pack2(S[2 * s][0], S[2 * s][1]), pack2(S[2 * s][2], S[2 * s][3]),
-                          pack2(S[2 * s + 1][0], S[2 * s + 1][1]), pack2(S[2 * s + 1][2], S[2 * s + 1][3])};
-        }
-        if (16 * w < nrows) {
+        for (int s = 0; s < 4; ++s)
+          sp[s] = u32x4{pack2(S[2 * s][0], S[2 * s][1]), pack2(S[2 * s][2], S[2 * s][3]),
+                        pack2(S[2 * s + 1][0], S[2 * s + 1][1]), pack2(S[2 * s + 1][2], S[2 * s + 1][3])};
+        if (w < 3 && 16 * w < nrows) {
 #pragma unroll
           for (int s = 0; s < 4; ++s) kop[s] = row16(sh.kr[s >> 1], 16 * w, s & 1, r16, g);
         }
@@ -417,13 +418,11 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
             u32x4 qop[4];
 #pragma unroll
             for (int s = 0; s < 4; ++s) qop[s] = row16(sh.qr[s >> 1], 16 * tt, s & 1, r16, g);
-            if (have_state) {
 #pragma unroll
-              for (int s = 0; s < 4; ++s) y[tt] = mfma16(sp[s], qop[s], y[tt]);
-            }
+            for (int s = 0; s < 4; ++s) y[tt] = mfma16(sp[s], qop[s], y[tt]);
             // scores^T tile (u, tt): kr_u . qr_t times 2^min(cs_t - cs_u, 0), strictly
-            // causal (mamba_fused.py:144-146). Tile u = w, except that wave 3 takes
-            // (0, 3) from wave 0.
+            // causal (mamba_fused.py:144-146). Tiles u = w, wave 2 also (3, 3):
+            // wave 3 forms the next chunk's controls meanwhile.
             auto score = [&](const u32x4 (&ko)[4], int u) {
               f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -441,12 +440,12 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
               *reinterpret_cast<u32x2*>(sh.sc + rb_off(16 * tt + r16, 4 * u + g)) =
                   u32x2{pack2(x[0], x[1]), pack2(x[2], x[3])};
             };
-            if (w <= tt && !(w == 0 && tt == 3)) score(kop, w);
-            if (w == 3 && tt == 3) {
-              u32x4 k0[4];
+            if (w < 3 && w <= tt) score(kop, w);
+            if (w == 2 && tt == 3) {
+              u32x4 k3[4];
 #pragma unroll
-              for (int s = 0; s < 4; ++s) k0[s] = row16(sh.kr[s >> 1], 0, s & 1, r16, g);
-              score(k0, 0);
+              for (int s = 0; s < 4; ++s) k3[s] = row16(sh.kr[s >> 1], 48, s & 1, r16, g);
+              score(k3, 3);
             }
           }
         }
@@ -513,7 +512,6 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
           a = mfma16(col16<true>(buf, u0, 0, r16, g), vb0, a);
           S[j] = mfma16(col16<true>(buf, u0, 1, r16, g), vb1, a);
         }
-        have_state = true;
       }
       if (more) {
         phase(th, c + 1);
