@@ -72,7 +72,7 @@ __device__ __forceinline__ u32x4 col16(const uint16_t* buf, int u0, int s, int r
 // RT: rotary pairs the cos/sin table holds (R <= RT).
 template <int RT>
 struct WideSmem {
-  static constexpr int TS = 2 * RT + 2;  // floats per table row
+  static constexpr int TS = 2 * RT + 4;  // floats per table row: 16-byte pieces of 8 rows on distinct banks
   uint16_t qr[2][64 * 64];  // bf16(rot(q + qb)), channels 0-63 and 64-127
   uint16_t kr[2][64 * 64];  // bf16(rot(k + kb) * s)
   uint16_t v[64 * 64];      // v
@@ -87,14 +87,22 @@ struct WideSmem {
   float skip[64];  // (q + qb).(k + kb) of each row
 };
 
-// Element i of a control, trapezoid or angle tensor. IN: 0 all three fp32, 1 all
-// bf16, 2 as the flag says.
+// IN: how the controls, trapezoid and angles are read. 0: all fp32, 1: all bf16,
+// both with the angles of eight neighbouring pairs in one aligned piece and byte
+// offsets below 2^32; 2: any mix, element by element.
 template <int IN>
-__device__ __forceinline__ float load_in(const void* base, int bf16, int i) {
-  if constexpr (IN == 2)
-    return ctl_value(base, bf16, i);
+__device__ __forceinline__ float load_in(const void* base, int bf16, uint32_t i) {
+  if constexpr (IN == 0)
+    return *reinterpret_cast<const float*>(static_cast<const char*>(base) + 4 * i);
+  else if constexpr (IN == 1)
+    return bf16_to_f32(*reinterpret_cast<const uint16_t*>(static_cast<const char*>(base) + 2 * i));
   else
-    return load_elem<IN == 1>(base, i);
+    return bf16 ? to_f32(static_cast<const bf16_t*>(base)[i]) : static_cast<const float*>(base)[i];
+}
+
+// 16 bytes of a bf16 row: the byte offset stays 32-bit (a uniform base plus one register).
+__device__ __forceinline__ u32x4 load_piece(const uint16_t* base, uint32_t i) {
+  return *reinterpret_cast<const u32x4_a8*>(reinterpret_cast<const char*>(base) + 2 * i);
 }
 
 // Raw 16-byte pieces of one row: channels 8 ng .. and 64 + 8 ng .. of q and k,
@@ -144,15 +152,13 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
   // lane-derived indices, rebuilt every chunk from an index the compiler cannot
   // see through: hoisted out of the walk, the LDS addresses they feed would
   // hold a register each and spill
-  int lane, r16, g, ng, row0, pi, sg;
+  int lane, r16, g, ng, row0;
   auto lane_indices = [&]() {
     lane = static_cast<int>(threadIdx.x & 63);
     asm volatile("" : "+v"(lane));
     r16 = lane & 15, g = lane >> 4;
     // rotation: rows 16 w + 8 i + row8 (i = 0, 1), eight lanes per row
     ng = lane & 7, row0 = 16 * w + row8_of_lane(lane);
-    // phase: lane = (pair of eight, segment of eight rows), pairs 32 i + 8 w + pi
-    pi = lane >> 3, sg = lane & 7;
   };
   lane_indices();
   const int T = P.T, R = P.R;
@@ -167,45 +173,49 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
 
   if (c1 > c0) {
     const int tlim = P.rev ? L : T;
-    const int roff = P.rev ? max(L - 1, 0) : 0;
     const int qh = h / P.group;
-    const uint16_t* qbase = P.q + b * P.q_sb + qh * P.q_sh - roff * P.q_st;
-    const uint16_t* kbase = P.k + b * P.k_sb + qh * P.k_sh - roff * P.k_st;
-    const uint16_t* vbase = P.v + b * P.v_sb + h * P.v_sh - roff * P.v_st;
-    const uint16_t* zbase = P.z + b * P.z_sb + h * P.z_sh - roff * P.z_st;
-    const int dto = b * P.d_sb + h * P.d_sh - roff * P.d_st;
-    const int ado = b * P.a_sb + h * P.a_sh - roff * P.a_st;
-    const int trb = b * P.r_sb + h * P.r_sh - roff * P.r_st;
-    const int gbase = b * P.g_sb + h * P.g_sh - roff * P.g_st;
-    const int obase = b * P.o_sb + h * P.o_sh - roff * P.o_st;
+    // rows of the unit: step t is row t, or L - 1 - t reversed (the time strides
+    // come negated then)
+    const uint16_t* qbase = P.q + (b * P.q_sb + qh * P.q_sh);
+    const uint16_t* kbase = P.k + (b * P.k_sb + qh * P.k_sh);
+    const uint16_t* vbase = P.v + (b * P.v_sb + h * P.v_sh);
+    const uint16_t* zbase = P.z + (b * P.z_sb + h * P.z_sh);
+    auto in_base = [&](const void* p, bool bf16, int off) -> const void* {
+      return static_cast<const char*>(p) + static_cast<int64_t>(off) * (IN == 1 || (IN == 2 && bf16) ? 2 : 4);
+    };
+    const bool ang16 = P.angles_dtype == TF_BFLOAT16;
+    const void* dtp = in_base(P.dt, P.ctl_bf16, b * P.d_sb + h * P.d_sh);
+    const void* adp = in_base(P.adt, P.ctl_bf16, b * P.a_sb + h * P.a_sh);
+    const void* trp = in_base(P.trap, P.trap_bf16, b * P.r_sb + h * P.r_sh);
+    const void* agp = in_base(P.angles, ang16, b * P.g_sb + h * P.g_sh);
+    const uint32_t q_st = abs(P.q_st), k_st = abs(P.k_st), v_st = abs(P.v_st), z_st = abs(P.z_st);
+    const uint32_t d_st = abs(P.d_st), a_st = abs(P.a_st), r_st = abs(P.r_st), g_st = abs(P.g_st);
+    auto row_of = [&](int t) -> uint32_t { return P.rev ? L - 1 - t : t; };
+    const int obase = b * P.o_sb + h * P.o_sh - (P.rev ? L - 1 : 0) * P.o_st;
     const float step_bias = P.ctl_raw ? P.dt_bias[h] : 0.f;
     const float skip_d = MODE == 0 ? P.d[h] : 0.f;
-    const int ang16 = P.angles_dtype == TF_BFLOAT16;
-
     auto load_rows = [&](int c, WideRow (&x)[2]) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const int t = min(c * kChunk + row0 + 8 * i, L - 1);
-        const uint16_t* kp = kbase + t * P.k_st + 8 * ng;
-        x[i].k[0] = *reinterpret_cast<const u32x4_a8*>(kp);
-        x[i].k[1] = *reinterpret_cast<const u32x4_a8*>(kp + 64);
-        x[i].v = *reinterpret_cast<const u32x4_a8*>(vbase + t * P.v_st + 8 * ng);
+        const uint32_t rr = row_of(min(c * kChunk + row0 + 8 * i, L - 1));
+        x[i].k[0] = load_piece(kbase, rr * k_st + 8 * ng);
+        x[i].k[1] = load_piece(kbase, rr * k_st + 8 * ng + 64);
+        x[i].v = load_piece(vbase, rr * v_st + 8 * ng);
         if constexpr (MODE == 0) {
-          const uint16_t* qp = qbase + t * P.q_st + 8 * ng;
-          x[i].q[0] = *reinterpret_cast<const u32x4_a8*>(qp);
-          x[i].q[1] = *reinterpret_cast<const u32x4_a8*>(qp + 64);
+          x[i].q[0] = load_piece(qbase, rr * q_st + 8 * ng);
+          x[i].q[1] = load_piece(qbase, rr * q_st + 8 * ng + 64);
         }
       }
     };
     // controls: wave 3, lane = row; rows clamped to ones that exist
     auto load_ctl = [&](int c) {
-      const int tc = min(c * kChunk + lane, L - 1), tn = min(c * kChunk + lane + 1, tlim - 1);
+      const uint32_t rc = row_of(min(c * kChunk + lane, L - 1)), rn = row_of(min(c * kChunk + lane + 1, tlim - 1));
       PipeCtl x;
-      x.dt = load_in<IN>(P.dt, P.ctl_bf16, dto + tc * P.d_st);
-      x.dn = load_in<IN>(P.dt, P.ctl_bf16, dto + tn * P.d_st);
-      x.adt = load_in<IN>(P.adt, P.ctl_bf16, ado + tc * P.a_st);
-      x.tr = load_in<IN>(P.trap, P.trap_bf16, trb + tc * P.r_st);
-      x.tn = load_in<IN>(P.trap, P.trap_bf16, trb + tn * P.r_st);
+      x.dt = load_in<IN>(dtp, P.ctl_bf16, rc * d_st);
+      x.dn = load_in<IN>(dtp, P.ctl_bf16, rn * d_st);
+      x.adt = load_in<IN>(adp, P.ctl_bf16, rc * a_st);
+      x.tr = load_in<IN>(trp, P.trap_bf16, rc * r_st);
+      x.tn = load_in<IN>(trp, P.trap_bf16, rn * r_st);
       return x;
     };
     float seg_log2 = 0.f;
@@ -219,60 +229,76 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
       sh.gam[cb][lane] = rc.gam;
       if (lane == 0) sh.tot[cb] = rc.tot;
     };
-    auto load_angles = [&](int c, float (&th)[PI][8]) {
+    // phase: lane = row, pairs 32 i + 8 w + j of wave w (raw angles: eight per row)
+    typedef float Angles[PI][8];
+    auto load_angles = [&](int c, Angles& th) {
+      const uint32_t rr = row_of(min(c * kChunk + lane, L - 1));
 #pragma unroll
       for (int i = 0; i < PI; ++i) {
-        const int pair = 32 * i + 8 * w + pi;
-        const int col = gbase + (pair < R ? pair : 0) * P.g_sr;
-        if (32 * i + 8 * w < R) {  // wave-uniform
+        const int p0 = 32 * i + 8 * w;
+        if (p0 < R) {  // wave-uniform
+          if constexpr (IN == 0) {
+            const char* p = static_cast<const char*>(agp) + 4 * (rr * g_st + p0);
+            const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 16);
+            th[i][0] = x.x, th[i][1] = x.y, th[i][2] = x.z, th[i][3] = x.w;
+            th[i][4] = y.x, th[i][5] = y.y, th[i][6] = y.z, th[i][7] = y.w;
+          } else if constexpr (IN == 1) {
+            // kept packed until used: four registers
+            const u32x4 x = *reinterpret_cast<const u32x4*>(static_cast<const char*>(agp) + 2 * (rr * g_st + p0));
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-            th[i][j] = load_in<IN>(P.angles, ang16, col + min(c * kChunk + 8 * sg + j, L - 1) * P.g_st);
+            for (int j = 0; j < 4; ++j) th[i][j] = __uint_as_float(x[j]);
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              th[i][j] = load_in<IN>(agp, ang16, rr * g_st + (p0 + j < R ? p0 + j : 0) * P.g_sr);
+          }
         }
       }
     };
-    uint32_t carry[PI];  // phase entering the chunk, 2^-32 revolutions
+    uint32_t carry[PI][8];  // phase entering the chunk, 2^-32 revolutions (wave-uniform)
 #pragma unroll
     for (int i = 0; i < PI; ++i) {
-      carry[i] = 0;
-      if (MODE == 0 && P.G > 1) {
-        // the wrapping sum of the preceding segments' phase sums
-        const int pair = 32 * i + 8 * w + pi;
+      uint32_t incl = 0;
+      if (MODE == 0 && seg > 0) {
+        // the wrapping sum of the preceding segments' phase sums: lane = (pair, eighth)
+        const int pair = 32 * i + 8 * w + (lane >> 3);
         uint32_t part = 0;
         if (pair < R)
-          for (int s = sg; s < seg; s += 8) part += P.phase_fx[(static_cast<size_t>(it.unit) * P.G + s) * RT + pair];
-        const uint32_t incl = group_scan_dpp<8>(part, lane);
-        carry[i] = __shfl(incl, lane | 7, 64);
+          for (int s = lane & 7; s < seg; s += 8) part += P.phase_fx[(static_cast<size_t>(it.unit) * P.G + s) * RT + pair];
+        incl = group_scan_dpp<8>(part, lane);
       }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        carry[i][j] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 8 * j + 7));
     }
-    auto phase = [&](const float (&th)[PI][8], int c) {
-      const float* dts = &sh.dt[c & 1][8 * sg];
-      const float4 da = *reinterpret_cast<const float4*>(dts), db = *reinterpret_cast<const float4*>(dts + 4);
-      const float dt[8] = {da.x, da.y, da.z, da.w, db.x, db.y, db.z, db.w};
+    auto phase = [&](const Angles& th, int c) {
+      const float dt = sh.dt[c & 1][lane];
 #pragma unroll
       for (int i = 0; i < PI; ++i) {
-        if (32 * i + 8 * w < R) {
-          uint32_t loc[8], run = 0;
+        const int p0 = 32 * i + 8 * w;
+        if (p0 < R) {
+          float* tg = &sh.trig[lane * TS + 2 * p0];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            run += phase_inc(th[i][j], dt[j]);
-            loc[j] = run;
-          }
-          const uint32_t incl = group_scan_dpp<8>(run, lane);
-          const uint32_t base = carry[i] + (incl - run);
-          const int pair = 32 * i + 8 * w + pi;
-          if (pair < R) {
-            float* tg = &sh.trig[8 * sg * TS + 2 * pair];
+          for (int j = 0; j < 8; j += 2) {
+            float2 x[2];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              float2 x = phase_trig(base + loc[j]);
+            for (int k = 0; k < 2; ++k) {
+              float a;
+              if constexpr (IN == 1)
+                a = k == 0 ? lo_f(__float_as_uint(th[i][j / 2])) : hi_f(__float_as_uint(th[i][j / 2]));
+              else
+                a = th[i][j + k];
+              const uint32_t incl = wave_scan_u32(phase_inc(a, dt));
+              x[k] = phase_trig(carry[i][j + k] + incl);
               // an angle that is not a number makes its row (and with it every
               // later one) not a number; fixed point alone would lose it
-              x.x = th[i][j] == th[i][j] ? x.x : th[i][j];
-              *reinterpret_cast<float2*>(tg + j * TS) = x;
+              x[k].x = a == a ? x[k].x : a;
+              carry[i][j + k] += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), 63));
+              // pairs that do not rotate turn by the identity
+              if (IN == 2 && p0 + j + k >= R) x[k] = make_float2(1.f, 0.f);
             }
+            *reinterpret_cast<float4*>(tg + 2 * j) = make_float4(x[0].x, x[0].y, x[1].x, x[1].y);
           }
-          carry[i] += __shfl(incl, lane | 7, 64);
         }
       }
     };
@@ -350,7 +376,7 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
     // the start's loads, then chunk c0's controls and phase
     WideRow rows[2];
     PipeCtl ctl = {};
-    float th[PI][8];
+    Angles th;
     if (w == 3) ctl = load_ctl(c0);
     load_angles(c0, th);
     load_rows(c0, rows);
@@ -362,8 +388,8 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
 #pragma unroll
       for (int j = 0; j < 8; ++j) S[j] = __builtin_bit_cast(f32x4, rec[j * kWideThreads]);
     }
-    // pairs that do not rotate, up to the end of the last rotating piece
-    for (int e = 64 * R + static_cast<int>(threadIdx.x); e < 64 * ((R + 31) & ~31); e += kWideThreads)
+    // pairs that no wave forms, up to the end of the last rotating piece
+    for (int e = 64 * ((R + 7) & ~7) + static_cast<int>(threadIdx.x); e < 64 * ((R + 31) & ~31); e += kWideThreads)
       *reinterpret_cast<float2*>(&sh.trig[(e & 63) * TS + 2 * (e >> 6)]) = make_float2(1.f, 0.f);
     if (threadIdx.x < 128) {
       sh.kb[threadIdx.x] = P.kb[h * 128 + threadIdx.x];
@@ -393,8 +419,9 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
       if constexpr (MODE == 0) {
 #pragma unroll
         for (int tt = 0; tt < 4; ++tt) {
-          const int t = min(c * kChunk + 16 * tt + r16, L - 1);
-          zr[tt] = *reinterpret_cast<const u32x2*>(zbase + t * P.z_st + 16 * w + 4 * g);
+          const uint32_t rr = row_of(min(c * kChunk + 16 * tt + r16, L - 1));
+          zr[tt] = *reinterpret_cast<const u32x2*>(reinterpret_cast<const char*>(zbase) +
+                                                   2 * (rr * z_st + 16 * w + 4 * g));
         }
       }
       if (more) load_rows(c + 1, rows);
@@ -529,7 +556,9 @@ __global__ __launch_bounds__(kWideThreads, RT == 32 ? 2 : 1) void mamba_wide_ker
       if (threadIdx.x == 0) P.seg_decay[it.rec] = seg_log2;
 #pragma unroll
       for (int i = 0; i < PI; ++i)
-        if (sg == 0) P.phase_fx[static_cast<size_t>(it.rec) * RT + 32 * i + 8 * w + pi] = carry[i];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (lane == j) P.phase_fx[static_cast<size_t>(it.rec) * RT + 32 * i + 8 * w + j] = carry[i][j];
     }
   }
   if constexpr (MODE == 0) {
@@ -652,9 +681,16 @@ int launch_wide(const tf_mamba_args& a, hipStream_t stream) {
   const int64_t items = static_cast<int64_t>(P.units) * P.G;
   P.xcd_per = (items % 8 == 0 && items >= 64) ? static_cast<int>(items / 8) : 0;
   const bool ang16 = P.angles_dtype == TF_BFLOAT16;
+  // angles in aligned pieces of eight pairs, every byte offset of the 32-bit
+  // operands below 2^32
+  bool pieces = a.rotary % 8 == 0 && P.g_sr == 1 && aligned(a.angles, 16);
+  for (int i = 0; i < 3; ++i) pieces = pieces && a.angles_stride[i] % 8 == 0;
+  const int64_t span = std::max({a.time * a.angles_stride[1], a.time * a.dt_stride[2], a.time * a.adt_stride[2],
+                                 a.time * a.trap_stride[2]});
+  pieces = pieces && span < (int64_t(1) << 29);
   if (a.rotary > 32) return launch_wide_kernel<64, 2>(P, stream);
-  if (!P.ctl_bf16 && !P.trap_bf16 && !ang16) return launch_wide_kernel<32, 0>(P, stream);
-  if (P.ctl_bf16 && P.trap_bf16 && ang16) return launch_wide_kernel<32, 1>(P, stream);
+  if (pieces && !P.ctl_bf16 && !P.trap_bf16 && !ang16) return launch_wide_kernel<32, 0>(P, stream);
+  if (pieces && P.ctl_bf16 && P.trap_bf16 && ang16) return launch_wide_kernel<32, 1>(P, stream);
   return launch_wide_kernel<32, 2>(P, stream);
 }
 
