@@ -4,7 +4,9 @@
 every ``csrc/*.hip`` file becomes an object under ``_build/`` and the objects
 are linked into ``trifusion_amd/libtrifusion_amd.so``, which ``_lib.py`` loads
 with ctypes. The library exports only the ``extern "C"`` entry points declared
-in ``include/trifusion_amd.h``.
+in ``include/trifusion_amd.h``. ``csrc/torch_ops.cpp``, host code that binds
+operators to torch's dispatcher, becomes ``trifusion_amd/libtrifusion_torch.so``
+beside it.
 """
 
 import os
@@ -20,6 +22,7 @@ CSRC_DIR = PROJECT_DIR / "csrc"
 INCLUDE_DIR = REPO_DIR / "include"
 BUILD_DIR = PROJECT_DIR / "_build"
 LIB_PATH = PACKAGE_DIR / "libtrifusion_amd.so"
+TORCH_LIB_PATH = PACKAGE_DIR / "libtrifusion_torch.so"
 ARCH = "gfx950"
 
 # Packed-fp32 VALU forms are disabled for all device code; hipcc -O3 would
@@ -73,7 +76,28 @@ def build_library(verbose=False, jobs=None):
     if proc.returncode != 0:
         raise RuntimeError("link failed:\n" + proc.stdout + proc.stderr)
     os.replace(tmp, LIB_PATH)
+    _build_torch_library(hipcc)
     return LIB_PATH
+
+
+def _build_torch_library(hipcc):
+    """Compile and link the operator bindings against the installed torch and the
+    library built just before (found at run time beside them)."""
+    import torch
+
+    base = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc).resolve().parents[1]
+    tmp = TORCH_LIB_PATH.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", str(INCLUDE_DIR),
+           "-isystem", str(base / "include"), "-isystem", str(base / "include/torch/csrc/api/include"),
+           "-isystem", str(rocm / "include"), str(CSRC_DIR / "torch_ops.cpp"), "-o", str(tmp),
+           "-L", str(base / "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-L", str(PACKAGE_DIR),
+           f"-l:{LIB_PATH.name}", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("g++ failed for torch_ops.cpp:\n" + proc.stdout + proc.stderr)
+    os.replace(tmp, TORCH_LIB_PATH)
 
 
 if __name__ == "__main__":

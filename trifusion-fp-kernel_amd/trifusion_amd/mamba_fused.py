@@ -45,7 +45,9 @@ def _shape_error(message):
 
 def build_args(q, k, v, adt, dt, trap, qb, kb, angles, d, z, out, lengths=None, variant="auto", reverse=False,
                dt_bias=None, a_floor=1e-4, q_norm=None, k_norm=None, norm_eps=1e-5):
-    """Validate the operands and pack them into a ``tf_mamba_args`` struct."""
+    """Validate the operands and pack them into a ``tf_mamba_args`` struct, for callers
+    of the C entries (the operator's own kernel does the same natively,
+    ``csrc/torch_ops.cpp``)."""
     what = "fused_mamba"
     for name, t in (("q", q), ("k", k), ("v", v), ("z", z), ("angles", angles)):
         if t.dim() != 4:
@@ -140,28 +142,6 @@ def build_args(q, k, v, adt, dt, trap, qb, kb, angles, d, z, out, lengths=None, 
     return a
 
 
-def launch(q, k, v, adt, dt, trap, qb, kb, angles, d, z, out, lengths=None, variant="auto", reverse=False,
-           dt_bias=None, a_floor=1e-4, q_norm=None, k_norm=None, norm_eps=1e-5):
-    """Validate, then enqueue ``tf_fused_mamba`` on the current stream (the CUDA
-    kernel of the ``trifusion_amd::fused_mamba`` operator); returns ``out``."""
-    lib = _lib.load()
-    args = build_args(q, k, v, adt, dt, trap, qb, kb, angles, d, z, out, lengths, variant, reverse, dt_bias, a_floor,
-                      q_norm, k_norm, norm_eps)
-    # Long sequences over few (batch, head) units run chunk-parallel on scratch
-    # the library sizes; it comes from torch's caching allocator (the graph's
-    # private pool under capture), the C side never allocates.
-    need = lib.tf_fused_mamba_workspace_size(ctypes.byref(args))
-    if need < 0:
-        _lib.check(-need, "fused_mamba")
-    workspace = None
-    if need > 0:
-        workspace = torch.empty(need, dtype=torch.uint8, device=v.device)
-        args.workspace = workspace.data_ptr()
-        args.workspace_bytes = need
-    _lib.check(lib.tf_fused_mamba(ctypes.byref(args), _lib.stream_of(v)), "fused_mamba")
-    return out
-
-
 def fused_mamba(
     q,
     k,
@@ -200,7 +180,7 @@ def fused_mamba(
     del warps
     ext = (lengths, variant, bool(reverse), dt_bias, float(a_floor), q_norm, k_norm, float(norm_eps))
     if out is None:
-        return ops.fused_mamba(q, k, v, adt, dt, trap, qb, kb, angles, d, z, *ext)
+        return ops.fused_mamba.default(q, k, v, adt, dt, trap, qb, kb, angles, d, z, *ext)
     return ops.fused_mamba.out(q, k, v, adt, dt, trap, qb, kb, angles, d, z, *ext, out=out)
 
 

@@ -4,7 +4,8 @@ Every compute entry point of ``include/trifusion_amd.h`` is registered with
 ``torch.library`` in the ``trifusion_amd`` namespace:
 
 * a CUDA kernel (ROCm devices dispatch through the CUDA key) that validates
-  the operands and calls the C entry on the current stream;
+  the operands and calls the C entry on the current stream (for
+  ``fused_mamba`` a native one, ``csrc/torch_ops.cpp``);
 * a Meta kernel giving output shapes and dtypes, so the operators trace under
   fake tensors (``torch.compile``, ``torch.export``) without a device;
 * a CPU kernel that raises: there is no CPU path by design.
@@ -17,6 +18,8 @@ operator layer is the torch-native form of that launch.
 """
 
 import torch
+
+from .build import TORCH_LIB_PATH
 
 NAMESPACE = "trifusion_amd"
 
@@ -101,23 +104,6 @@ OPERATORS = tuple(_SCHEMAS)
 
 
 # ---- CUDA kernels: the ctypes launches (imported lazily: those modules call these operators) ----
-
-
-def _cuda_fused_mamba(q, k, v, adt, dt, trap, qb, kb, angles, d, z, lengths=None, variant="auto", reverse=False,
-                      dt_bias=None, a_floor=1e-4, q_norm=None, k_norm=None, norm_eps=1e-5):
-    from .mamba_fused import launch
-
-    out = torch.empty_like(v, memory_format=torch.contiguous_format)
-    return launch(q, k, v, adt, dt, trap, qb, kb, angles, d, z, out, lengths, variant, reverse, dt_bias, a_floor,
-                  q_norm, k_norm, norm_eps)
-
-
-def _cuda_fused_mamba_out(q, k, v, adt, dt, trap, qb, kb, angles, d, z, lengths=None, variant="auto", reverse=False,
-                          dt_bias=None, a_floor=1e-4, q_norm=None, k_norm=None, norm_eps=1e-5, *, out):
-    from .mamba_fused import launch
-
-    return launch(q, k, v, adt, dt, trap, qb, kb, angles, d, z, out, lengths, variant, reverse, dt_bias, a_floor,
-                  q_norm, k_norm, norm_eps)
 
 
 def _cuda_rms_norm(x, weight, eps=1e-5, out_dtype=None):
@@ -419,9 +405,23 @@ def _no_cpu(name):
     return kernel
 
 
+# operators whose CUDA kernel is native (csrc/torch_ops.cpp)
+_NATIVE = None
+
+
+def _not_built(name):
+    def kernel(*args, **kwargs):
+        raise RuntimeError(
+            f"{NAMESPACE}::{name}: native operator library not built ({TORCH_LIB_PATH}); run "
+            "`python -c 'import __graft_entry__ as g; g.build()'` from the repository root"
+        )
+
+    return kernel
+
+
 _KERNELS = {
-    "fused_mamba": (_cuda_fused_mamba, _meta_fused_mamba),
-    "fused_mamba.out": (_cuda_fused_mamba_out, _meta_fused_mamba_out),
+    "fused_mamba": (_NATIVE, _meta_fused_mamba),
+    "fused_mamba.out": (_NATIVE, _meta_fused_mamba_out),
     "rms_norm": (_cuda_rms_norm, _meta_rms_norm),
     "add_rms_norm": (_cuda_add_rms_norm, _meta_add_rms_norm),
     "add": (_cuda_add, _meta_add),
@@ -450,8 +450,14 @@ _LIBRARY = torch.library.Library(NAMESPACE, "DEF")
 for _name, _schema in _SCHEMAS.items():
     _LIBRARY.define(_schema)
     _cuda, _meta = _KERNELS[_name]
-    _LIBRARY.impl(_name, _cuda, "CUDA")
+    if _cuda is not _NATIVE:
+        _LIBRARY.impl(_name, _cuda, "CUDA")
+    elif not TORCH_LIB_PATH.exists():
+        _LIBRARY.impl(_name, _not_built(_name), "CUDA")
     _LIBRARY.impl(_name, _meta, "Meta")
     _LIBRARY.impl(_name, _no_cpu(_name), "CPU")
+
+if TORCH_LIB_PATH.exists():
+    torch.ops.load_library(str(TORCH_LIB_PATH))
 
 ops = getattr(torch.ops, NAMESPACE)
