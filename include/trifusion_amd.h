@@ -567,6 +567,16 @@ int tf_front_lengths(const int64_t *sample_lengths, int64_t *out, int64_t batch,
 int tf_grids(const int64_t *lengths, void *mask, int64_t *low_lengths, void *low_mask, int64_t *left,
              int64_t *right, float *alpha, int64_t batch, int64_t time, void *stream);
 
+/*
+ * Log power spectrogram of the front end in one pass (src/trifusion_l4/front.py:46-90):
+ * tf_mask_audio, the centred 512-point STFT (hop 160, zero padding, a 400-point
+ * window in the middle of the frame) and tf_log_power, with no waveform copy or
+ * spectrum written. audio fp32 contiguous [B, C, N], window fp32 [400], lengths and
+ * channels int64 [B]; y fp32 contiguous [B, N / 160 + 1, 257].
+ */
+int tf_log_spectrogram(const float *audio, const float *window, const int64_t *lengths, const int64_t *channels,
+                       float *y, int64_t batch, int64_t chans, int64_t samples, void *stream);
+
 /* Library version string (static storage). */
 const char *tf_version(void);
 

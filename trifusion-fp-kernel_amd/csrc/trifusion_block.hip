@@ -314,6 +314,38 @@ __global__ __launch_bounds__(256) void bands_kernel(const T* __restrict__ x, T* 
   y[i] = from_f32<T>(acc / static_cast<float>(end - start));
 }
 
+// As bands_kernel for channels-last maps (sc == 1), eight neighbouring channels per
+// thread: 16- or 32-byte loads, the same sums in the same order. Channels one at a
+// time, 2-byte loads and an index division per element took 13.3 us a call on the
+// front end's maps of 8 stereo clips of 8 s; this one takes 6.1.
+template <typename T>
+__global__ __launch_bounds__(256) void bands_vec_kernel(const T* __restrict__ x, T* __restrict__ y, int Tn, int F, int C8,
+                                                        int64_t total, int64_t sb, int64_t st, int64_t sf) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const int c8 = static_cast<int>(i % C8);
+  const int band = static_cast<int>((i / C8) % 8);
+  const int64_t bt = i / (static_cast<int64_t>(C8) * 8);
+  const int t = static_cast<int>(bt % Tn);
+  const int64_t b = bt / Tn;
+  const int start = band * F / 8;
+  const int end = ((band + 1) * F + 7) / 8;
+  const T* src = x + b * sb + 8 * c8 + t * st;
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+#pragma unroll 4
+  for (int f = start; f < end; ++f) {
+    float v[8];
+    load8v(src + f * sf, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] += v[e];
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] /= static_cast<float>(end - start);
+  store8v(y + 8 * i, acc);
+}
+
 // s = mask[row] ? x + a * (2 sigmoid(g)) : 0 (fp32), y = s rsqrt(mean(s^2) + eps) w
 // in fp32 (kernels/native.py:_norm MODE 1 via evidence_norm). One wave per row;
 // the second pass recomputes s from the (now cached) row.
@@ -531,6 +563,19 @@ extern "C" int tf_bands(const void* x, int32_t dtype, const int64_t* strides, vo
   const int64_t total = batch * time * 8 * chans;
   if (total == 0) return TF_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // whole aligned pieces of eight channels
+  const bool vec = strides[1] == 1 && chans % 8 == 0 && strides[0] % 8 == 0 && strides[2] % 8 == 0 &&
+                   strides[3] % 8 == 0 && tf::aligned16(x) && tf::aligned16(y);
+  if (vec && (dtype == TF_FLOAT32 || dtype == TF_BFLOAT16)) {
+    auto launch = [&](auto* p) {
+      using T = std::remove_pointer_t<decltype(p)>;
+      hipLaunchKernelGGL(tf::bands_vec_kernel<T>, dim3(tf::nblocks(total / 8, 256)), dim3(256), 0, s,
+                         static_cast<const T*>(x), static_cast<T*>(y), static_cast<int>(time), static_cast<int>(freq),
+                         static_cast<int>(chans / 8), total / 8, strides[0], strides[2], strides[3]);
+      return tf::launch_status();
+    };
+    return dtype == TF_FLOAT32 ? launch(static_cast<float*>(nullptr)) : launch(static_cast<tf::bf16_t*>(nullptr));
+  }
   TF_DISPATCH(dtype, T,
               hipLaunchKernelGGL(tf::bands_kernel<T>, dim3(tf::nblocks(total, 256)), dim3(256), 0, s,
                                  static_cast<const T*>(x), static_cast<T*>(y), static_cast<int>(time),

@@ -159,6 +159,7 @@ _SIGNATURES = {
         [c_ptr, ctypes.POINTER(c_i64), c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_i64, c_i64, c_ptr],
         c_i32,
     ),
+    "tf_log_spectrogram": ([c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_ptr], c_i32),
     "tf_front_lengths": ([c_ptr, c_ptr, c_i64, c_i64, ctypes.POINTER(c_i64), c_ptr], c_i32),
     "tf_grids": ([c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_ptr], c_i32),
     "tf_version": ([], ctypes.c_char_p),

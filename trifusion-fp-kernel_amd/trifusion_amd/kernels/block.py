@@ -671,6 +671,28 @@ def launch_log_power(spec, channels, sample_lengths, hop):
     return y
 
 
+def log_spectrogram(audio, window, lengths, channels):
+    """``[B, C, N]`` waveform -> fp32 ``[B, N // 160 + 1, 257]``: the centred 512-point
+    STFT every 160 samples under a 400-point window, its power summed over each
+    clip's channels, ``log(1e-6 + power / channels)``; samples and frames past each
+    length count as 0 (``trifusion_amd::log_spectrogram``)."""
+    return ops.log_spectrogram(audio, window, lengths, channels)
+
+
+def launch_log_spectrogram(audio, window, lengths, channels):
+    lib = _lib.load()
+    _lib.require_cuda(audio, window, lengths, channels, what="log_spectrogram")
+    if audio.dim() != 3 or tuple(window.shape) != (400,):
+        raise ValueError("log_spectrogram: audio must be [B, C, N] and the window [400]")
+    x = audio.float().contiguous()
+    b, c, n = x.shape
+    y = torch.empty((b, n // 160 + 1, 257), device=x.device, dtype=torch.float32)
+    status = lib.tf_log_spectrogram(x.data_ptr(), window.float().contiguous().data_ptr(), _lengths(lengths).data_ptr(),
+                                    _lengths(channels).data_ptr(), y.data_ptr(), b, c, n, _lib.stream_of(x))
+    _lib.check(status, "log_spectrogram")
+    return y
+
+
 def front_lengths(sample_lengths, hop=160, strides=(1, 2, 2)):
     """int64 ``[4, B]``: frames ``n // hop + 1`` and the counts after each CNN stage
     (``trifusion_amd::front_lengths``)."""

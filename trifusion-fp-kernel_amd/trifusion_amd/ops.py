@@ -92,6 +92,7 @@ _SCHEMAS = {
     "query_read": "query_read(Tensor q, Tensor kv, Tensor key_lengths, int heads) -> Tensor",
     "mask_audio": "mask_audio(Tensor audio, Tensor lengths, Tensor channels) -> Tensor",
     "log_power": "log_power(Tensor spec, Tensor channels, Tensor sample_lengths, int hop) -> Tensor",
+    "log_spectrogram": "log_spectrogram(Tensor audio, Tensor window, Tensor lengths, Tensor channels) -> Tensor",
     "front_lengths": "front_lengths(Tensor sample_lengths, int hop, int[] strides) -> Tensor",
     "grids": "grids(Tensor lengths, int time) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)",
     "front_conv2": (
@@ -381,6 +382,10 @@ def _meta_log_power(spec, channels, sample_lengths, hop):
     return spec.new_empty((channels.shape[0], spec.shape[2], spec.shape[1]), dtype=torch.float32)
 
 
+def _meta_log_spectrogram(audio, window, lengths, channels):
+    return audio.new_empty((audio.shape[0], audio.shape[2] // 160 + 1, 257), dtype=torch.float32)
+
+
 def _meta_front_lengths(sample_lengths, hop, strides):
     return sample_lengths.new_empty((4, sample_lengths.shape[0]), dtype=torch.int64)
 
@@ -442,7 +447,8 @@ _KERNELS = {
         for name in ("depthwise_masked", "pool4", "rotary_qkv", "front_norm", "interpolate", "interpolate_rmsnorm",
                      "bands", "evidence_norm", "gated_concat", "front_conv1", "front_conv2", "block_pre",
                      "block_pre_add", "norm_silu", "glu_depthwise", "glu_norm_silu", "pooled_attention", "merge_gate",
-                     "evidence_down", "merge_conv", "query_read", "mask_audio", "log_power", "front_lengths", "grids")
+                     "evidence_down", "merge_conv", "query_read", "mask_audio", "log_power", "log_spectrogram",
+                     "front_lengths", "grids")
     },
 }
 

@@ -4,8 +4,8 @@ The reference model's layout and forward (``src/trifusion_l4/model.py``,
 ``front.py``, ``decoder.py``, ``masking.py``, ``attention.py``) with the same
 parameter names, so a checkpoint saved from either loads into the other:
 
-* ``Frontend``: log power STFT (``torch.stft``, 512-point, hop 160, Hann 400),
-  three CNN stages and 8 frequency bands (``tf_bands``) (``front.py:8-114``);
+* ``Frontend``: log power STFT (512-point, hop 160, Hann 400; ``tf_log_spectrogram``
+  on the GPU), three CNN stages and 8 frequency bands (``tf_bands``) (``front.py:8-114``);
   under bf16 autocast each stage is two fused kernels (``tf_front_conv1``: 3x3
   conv, channel RMSNorm, SiLU; ``tf_front_conv2``: 3x3 conv, RMSNorm, 1x1 skip
   conv, residual, SiLU), otherwise Conv2d with ``tf_front_norm``;
@@ -59,8 +59,7 @@ from .kernels.block import (
     pack_conv3x3,
     front_lengths,
     grids,
-    log_power,
-    mask_audio,
+    log_spectrogram,
     pooled_attention,
     query_read,
 )
@@ -215,14 +214,9 @@ class Frontend(nn.Module):
         when the caller has them)."""
         b, c, n = audio.shape
         if audio.is_cuda:
-            # masking and the log-power post-processing as one launch each around rocFFT
-            wave = mask_audio(audio, sample_lengths, channels)
-            with torch.autocast("cuda", enabled=False):
-                spec = torch.stft(wave, n_fft=512, hop_length=160, win_length=400, window=self.window.float(),
-                                  center=True, pad_mode="constant", return_complex=True)
             if frames is None:
                 frames = sample_lengths // 160 + 1
-            return log_power(spec, channels, sample_lengths, 160).unsqueeze(1), frames
+            return log_spectrogram(audio, self.window, sample_lengths, channels).unsqueeze(1), frames
         with torch.autocast("cuda", enabled=False):
             keep = time_mask(sample_lengths, n)[:, None, :] & (torch.arange(c, device=audio.device)[None, :]
                                                                < channels[:, None])[..., None]
