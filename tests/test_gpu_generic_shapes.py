@@ -89,3 +89,25 @@ def test_infinite_value_is_causal():
         assert not y[0, at, 0, 3].isfinite() and not y[0, at + 1 :, 0, 3].isfinite().any()
         rest = [i for i in range(64) if i != 3]
         assert max_rel(y[..., rest].cpu(), clean[..., rest].cpu()) <= 5e-6
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("b,t,h,n,p,r,lengths", [(1, 257, 2, 64, 64, 16, None), (3, 900, 4, 128, 64, 32, [900, 130, 0]),
+                                                 (2, 640, 1, 32, 32, 9, [385, 640]), (1, 1600, 3, 16, 32, 8, None)])
+def test_segments_match_serial_walk(b, t, h, n, p, r, lengths, reverse):
+    """Chunk-parallel (the operator brings scratch) against the serial walk (none given)
+    and the oracle: fp32 sums of the same terms, the carried state composed in
+    another order and its rotary rows turned once more per segment."""
+    args = clip_inputs(b, t, heads=h, head_dim=p, state=n, rotary=r, dtype=torch.float32, seed=t)
+    dev = on(args)
+    dl = None if lengths is None else torch.tensor(lengths, device=DEV)
+    serial = call(dev, torch.full((b, t, h, p), math.nan, device=DEV), dl, reverse)
+    out = torch.full((b, t, h, p), math.nan, device=DEV)
+    y = fused_mamba(*dev, out=out, lengths=dl, reverse=reverse)
+    assert max_rel(y.cpu(), serial.cpu()) <= 5e-6
+    hl = None if lengths is None else torch.tensor(lengths)
+    ref = (fused_mamba_reversed if reverse else fused_mamba_chunked)(*args, lengths=hl)
+    assert max_rel(y.cpu(), ref) <= 1e-5
+    if lengths is not None:
+        for i, length in enumerate(lengths):
+            assert not y[i, length:].any()

@@ -94,7 +94,7 @@ extern "C" int64_t tf_fused_mamba_workspace_size(const tf_mamba_args* a) {
   if (which < 0) return which;
   if (tf::empty(a)) return 0;
   if (which == TF_MAMBA_PIPE) return tf::pipe_workspace_bytes(*a);
-  return which == TF_MAMBA_MFMA ? tf::mfma_workspace_bytes(*a) : 0;
+  return which == TF_MAMBA_MFMA ? tf::mfma_workspace_bytes(*a) : tf::generic_workspace_bytes(*a);
 }
 
 extern "C" int tf_fused_mamba_static(const tf_mamba_args* a, void* stream) {
@@ -102,7 +102,14 @@ extern "C" int tf_fused_mamba_static(const tf_mamba_args* a, void* stream) {
   if (which < 0) return -which;
   if (tf::empty(a)) return TF_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (which == TF_MAMBA_GENERIC) return tf::launch_generic(*a, s);
+  if (which == TF_MAMBA_GENERIC) {
+    // its chunk-parallel form is not offered here: a long fp32 call's records
+    // would need more than the array holds, and the serial walk needs none
+    tf_mamba_args serial = *a;
+    serial.workspace = nullptr;
+    serial.workspace_bytes = 0;
+    return tf::launch_generic(serial, s);
+  }
   const int64_t need = which == TF_MAMBA_PIPE ? tf::pipe_workspace_bytes(*a) : tf::mfma_workspace_bytes(*a);
   tf_mamba_args local = *a;
   local.workspace = nullptr;

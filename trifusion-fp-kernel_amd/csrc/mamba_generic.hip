@@ -23,11 +23,16 @@
 //
 // What bounds it: the chain of one chunk, ~11 us at N = P = 64 of which the
 // products take ~4 (a SIMD's two waves share a 32-bit matrix unit), the rest
-// being the latency of controls, phase and rotation between barriers. B4 L400
-// H16 P64 N64, fp32: 80 us (2,155 us with contractions formed element by
-// element from LDS and one thread per phase pair); B1 L1600 H16 N128: 446 us
-// (13.2 ms). 32-bit offsets take the clip from 108 to 80 us against 64-bit ones
-// (fewer scalar registers spilled), so they are used wherever they fit.
+// being the latency of controls, phase and rotation between barriers. So few long
+// fp32 units run chunk-parallel: segment summaries (MODE 1: keys and values only),
+// a scan of their states, and walks of the segments. B4 L400 H16 P64 N64, fp32:
+// 80 us in one segment per unit, 63 us in three (2,155 us with contractions formed
+// element by element from LDS and one thread per phase pair); B1 L1600 H16 N128:
+// 446 and 104 us (13.2 ms). 32-bit offsets take the clip from 108 to 80 us against
+// 64-bit ones (fewer scalar registers spilled), so they are used wherever they fit.
+#include <algorithm>
+#include <type_traits>
+
 #include "mfma_tile.h"
 
 // Outside the contractions every product and sum is rounded on its own, as the
@@ -130,7 +135,19 @@ struct GenericParams {
   I q[4], k[4], v[4], z[4], g[4], o[4];  // [batch, time, head, element]
   I ad[3], dt[3], tr[3];                 // [batch, head, time]
   int qvec, kvec, vvec;                  // rows can be read four elements at a time
+  // chunk-parallel form: G segments per unit; per (unit, segment but the last) the
+  // state in the walk's registers' order, per (unit, segment) log2 decay and phase
+  // sums (revolutions, [G][64])
+  int G;
+  float4* state;
+  float* decay;
+  double* phase;
 };
+
+// First chunk of segment g of `chunks`, split as evenly as G segments allow.
+__device__ __forceinline__ int first_chunk(int chunks, int G, int g) {
+  return g * (chunks / G) + min(g, chunks % G);
+}
 
 template <int NT>
 struct GenericShared {
@@ -187,7 +204,9 @@ __device__ __forceinline__ void scatter16(void* p, int dtype, F&& off, const flo
 
 // NT: 32-channel tiles of the state dim. RP: phase pairs per wave (8 RP >= R).
 // ROUND: some operand is 16-bit, so the rounding points are not the identity.
-template <int NT, int RP, bool ROUND, typename I>
+// MODE 0: outputs of the unit's (or, P.G > 1, the segment's) chunks. MODE 1: the
+// segment's state from zero state and phase, its log2 decay and phase sums.
+template <int NT, int RP, bool ROUND, typename I, int MODE>
 __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericParams<I> P) {
   using Sm = GenericShared<NT>;
   constexpr int NS = Sm::NS, TS = Sm::TS, VS = Sm::VS, SS = Sm::SS;
@@ -195,6 +214,8 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
   const tf_mamba_args& a = P.a;
   const int h = blockIdx.x;
   const int b = blockIdx.y;
+  const int seg = blockIdx.z;
+  if (MODE == 1 && seg == P.G - 1) return;  // no segment starts from the last one's state
   const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int n_state = static_cast<int>(a.state);
   const int p_dim = static_cast<int>(a.head_dim);
@@ -222,7 +243,11 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
   const I tro = b * P.tr[0] + h * P.tr[1] - roff * P.tr[2];
 
   const float skip = a.d[h];
-  const int nchunks = (L + kChunk - 1) / kChunk;
+  const int total = (T + kChunk - 1) / kChunk;
+  const int nvalid = (L + kChunk - 1) / kChunk;
+  const int c0 = min(first_chunk(total, P.G, seg), nvalid);
+  const int nchunks = min(first_chunk(total, P.G, seg + 1), nvalid);  // the segment's chunks end here
+  const int unit = b * static_cast<int>(a.heads) + h;
   // output waves: rows 32 th .., columns 32 pt ..; state waves: tiles s, s + 4 of (n, p)
   const int PT = p_dim > 32 ? 2 : 1;
   const int th = (w & 3) >> 1, pt = w & 1;
@@ -239,7 +264,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
     const I r = min(t, L - 1);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      xq[j] = load_piece(a.q, a.q_dtype, qo + r * P.q[1], P.q[3], 4 * grp + 32 * j, n_state, P.qvec);
+      if (MODE == 0) xq[j] = load_piece(a.q, a.q_dtype, qo + r * P.q[1], P.q[3], 4 * grp + 32 * j, n_state, P.qvec);
       xk[j] = load_piece(a.k, a.k_dtype, ko + r * P.k[1], P.k[3], 4 * grp + 32 * j, n_state, P.kvec);
     }
 #pragma unroll
@@ -265,9 +290,40 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
 
   f32x16 state[2] = {zero16(), zero16()};  // state waves
   double carry[RP];             // phase entering the chunk, revolutions
+  float seg_log2 = 0.f;
 #pragma unroll
   for (int i = 0; i < RP; ++i) carry[i] = 0.0;
-  for (int e = static_cast<int>(threadIdx.x); e < kPMax * NS; e += kThreads) sh.st[e] = 0.f;
+  if (MODE == 0 && seg > 0 && nchunks > c0) {
+    // the phase and state entering the segment
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+      const int pair = w * RP + i, ln = static_cast<int>(threadIdx.x & 63);
+      double part = 0.0;
+      if (pair < rot)
+        for (int g = ln; g < seg; g += 64) part += P.phase[(static_cast<int64_t>(unit) * P.G + g) * 64 + pair];
+      const double sum = last_lane_f64(wave_scan_f64(part));
+      carry[i] = sum - __builtin_rint(sum);
+    }
+    const float4* rec = P.state + (static_cast<int64_t>(unit) * (P.G - 1) + seg - 1) * (NT * PT * 256);
+    if (w >= 4) {
+      const int ln = static_cast<int>(threadIdx.x & 63);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int tile = s_idx + 4 * i;
+        if (tile < NT * PT) {
+          const int sp = PT == 2 ? tile & 1 : 0, sn = PT == 2 ? tile >> 1 : tile;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const float4 x = rec[(tile * 4 + g) * 64 + ln];
+            state[i][4 * g] = x.x, state[i][4 * g + 1] = x.y, state[i][4 * g + 2] = x.z, state[i][4 * g + 3] = x.w;
+            *reinterpret_cast<float4*>(&sh.st[(32 * sp + (ln & 31)) * NS + 32 * sn + 8 * g + 4 * (ln >> 5)]) = x;
+          }
+        }
+      }
+    }
+  } else if (MODE == 0) {
+    for (int e = static_cast<int>(threadIdx.x); e < kPMax * NS; e += kThreads) sh.st[e] = 0.f;
+  }
   for (int e = static_cast<int>(threadIdx.x); e < Sm::NP; e += kThreads) {
     const bool on = e < n_state;
     sh.qb[e] = on ? a.qb[h * n_state + e] : 0.f;
@@ -275,9 +331,9 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
     sh.qw[e] = on && norm ? a.q_norm[e] : 0.f;
     sh.kw[e] = on && norm ? a.k_norm[e] : 0.f;
   }
-  if (nchunks > 0) load_chunk(0, static_cast<int>(threadIdx.x));
+  if (nchunks > c0) load_chunk(c0, static_cast<int>(threadIdx.x));
 
-  for (int c = 0; c < nchunks; ++c) {
+  for (int c = c0; c < nchunks; ++c) {
     const int t0 = c * kChunk;
     // lane-derived indices from a thread index the compiler cannot see through:
     // hoisted out of the loop, the addresses they feed would live across it
@@ -345,10 +401,11 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
         float sq = 0.f, sk = 0.f;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-          sq += xq[j].x * xq[j].x, sq += xq[j].y * xq[j].y, sq += xq[j].z * xq[j].z, sq += xq[j].w * xq[j].w;
+          if (MODE == 0)
+            sq += xq[j].x * xq[j].x, sq += xq[j].y * xq[j].y, sq += xq[j].z * xq[j].z, sq += xq[j].w * xq[j].w;
           sk += xk[j].x * xk[j].x, sk += xk[j].y * xk[j].y, sk += xk[j].z * xk[j].z, sk += xk[j].w * xk[j].w;
         }
-        rq = rsqrtf(group8_sum(sq) / static_cast<float>(n_state) + a.norm_eps);
+        if (MODE == 0) rq = rsqrtf(group8_sum(sq) / static_cast<float>(n_state) + a.norm_eps);
         rk = rsqrtf(group8_sum(sk) / static_cast<float>(n_state) + a.norm_eps);
       }
       const float scl = sh.scale[rrow];
@@ -356,6 +413,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
         const int n0 = 4 * grp + 32 * j;
+        if (MODE == 1) xq[j] = make_float4(0.f, 0.f, 0.f, 0.f);  // no query is formed
         float q[4] = {xq[j].x, xq[j].y, xq[j].z, xq[j].w}, k[4] = {xk[j].x, xk[j].y, xk[j].z, xk[j].w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -382,7 +440,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
           kv[e + 1] = rnd((k[e] * si + k[e + 1] * co) * scl, a.k_dtype);
         }
         const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        *reinterpret_cast<float4*>(&sh.qr[rrow * NS + n0]) = valid ? make_float4(qv[0], qv[1], qv[2], qv[3]) : z4;
+        if (MODE == 0) *reinterpret_cast<float4*>(&sh.qr[rrow * NS + n0]) = valid ? make_float4(qv[0], qv[1], qv[2], qv[3]) : z4;
         *reinterpret_cast<float4*>(&sh.kr[rrow * NS + n0]) = valid ? make_float4(kv[0], kv[1], kv[2], kv[3]) : z4;
       }
 #pragma unroll
@@ -397,7 +455,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
     // the gate rows of this chunk and the next chunk's operands, in flight over the products
     float zz[16];
     const bool late = t0 + 32 >= L;  // the chunk's second half has no valid row
-    const bool y_on = out_wave && !(late && th == 1);
+    const bool y_on = MODE == 0 && out_wave && !(late && th == 1);
     if (y_on) {
       // rows and columns clamped to ones that exist; masked at the store
       const I zc = zo + min(32 * pt + c32, p_dim - 1) * P.z[3];
@@ -417,7 +475,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
         inter = mfma_f32(xa.z, ya.z, inter);
         inter = mfma_f32(xa.w, ya.w, inter);
       }
-    } else if (w >= 4 && w < 7 && !(late && w > 4)) {
+    } else if (MODE == 0 && w >= 4 && w < 7 && !(late && w > 4)) {
       // strictly causal decayed scores, rounded to v's dtype (mamba_fused.py:144-146):
       // lane = t, values = u
       const int tt = w > 4 ? 1 : 0, uu = w > 5 ? 1 : 0;
@@ -487,10 +545,11 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
       const I oc = oo + p * P.o[3] + (t0 + 32 * th) * P.o[1];
       if (p < p_dim)
         scatter16(a.out, a.out_dtype, [&](int e) -> I { return oc + drow(e, hh) * P.o[1]; }, y2, count);
-    } else if (w >= 4 && c + 1 < nchunks) {
+    } else if (w >= 4 && (c + 1 < nchunks || (MODE == 1 && c + 1 < nvalid))) {
       // state update S <- S 2^tot + round_k(v 2^(tot-cs))^T kr (mamba_fused.py:150-152):
       // lane = p, values = n
       const float decay = sh.ecs[kChunk - 1];
+      seg_log2 += sh.cs[kChunk - 1];
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int tile = s_idx + 4 * i;
@@ -514,13 +573,123 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
     }
     __syncthreads();
   }
-  // rows past the valid prefix (the same rows in either direction)
-  const I st = rev ? -P.o[1] : P.o[1];
-  const I of = b * P.o[0] + h * P.o[2];
-  for (int t = L + w; t < T; t += kThreads / 64) {
-    const int p = static_cast<int>(threadIdx.x & 63);
-    if (p < p_dim) store_f32(a.out, a.out_dtype, of + t * st + p * P.o[3], 0.f);
+  if constexpr (MODE == 1) {
+    float4* rec = P.state + (static_cast<int64_t>(unit) * (P.G - 1) + seg) * (NT * PT * 256);
+    const int ln = static_cast<int>(threadIdx.x & 63);
+    if (w >= 4) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int tile = s_idx + 4 * i;
+        if (tile < NT * PT) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            rec[(tile * 4 + g) * 64 + ln] =
+                make_float4(state[i][4 * g], state[i][4 * g + 1], state[i][4 * g + 2], state[i][4 * g + 3]);
+        }
+      }
+      if (w == 4 && ln == 0) P.decay[static_cast<int64_t>(unit) * P.G + seg] = seg_log2;
+    }
+#pragma unroll
+    for (int i = 0; i < RP; ++i)
+      if (ln == 0 && w * RP + i < rot) P.phase[(static_cast<int64_t>(unit) * P.G + seg) * 64 + w * RP + i] = carry[i];
+  } else {
+    // rows past the valid prefix (the same rows in either direction)
+    const I st = rev ? -P.o[1] : P.o[1];
+    const I of = b * P.o[0] + h * P.o[2];
+    const int stop = min(first_chunk(total, P.G, seg + 1) * kChunk, T);
+    for (int t = max(first_chunk(total, P.G, seg) * kChunk, L) + w; t < stop; t += kThreads / 64) {
+      const int p = static_cast<int>(threadIdx.x & 63);
+      if (p < p_dim) store_f32(a.out, a.out_dtype, of + t * st + p * P.o[3], 0.f);
+    }
   }
+}
+
+// Replaces each unit's segment summaries by the states entering the next
+// segments: S_1 = d_0, S_{g+1} = S_g 2^dec_g + turn_g(d_g), where turn_g rotates
+// the rotary row pairs by the phase entering segment g (a summary is formed from
+// phase 0 at its segment's start, and is linear in the keys that phase turns).
+// Thread f of a unit takes float4 f of its records: channels n .. n + 3.
+template <typename I>
+__global__ __launch_bounds__(64) void generic_scan_kernel(const GenericParams<I> P, int kf4, int pt) {
+  constexpr int kBatch = 4;
+  const int slices = kf4 / 64;
+  const int unit = blockIdx.x / slices;
+  const int f = (blockIdx.x - unit * slices) * 64 + threadIdx.x;
+  const int tile = f >> 8, n = 32 * (pt == 2 ? tile >> 1 : tile) + 8 * ((f >> 6) & 3) + 4 * ((f >> 5) & 1);
+  const int G = P.G, rot = static_cast<int>(P.a.rotary), pair = n / 2;
+  float4* st = P.state + static_cast<int64_t>(unit) * (G - 1) * kf4 + f;
+  const float* dec = P.decay + static_cast<int64_t>(unit) * G;
+  const double* ph = P.phase + static_cast<int64_t>(unit) * G * 64 + pair;
+  float4 run = make_float4(0.f, 0.f, 0.f, 0.f);
+  double p0 = 0.0, p1 = 0.0;
+  for (int g0 = 0; g0 < G - 1; g0 += kBatch) {
+    float4 d[kBatch];
+    double s0[kBatch], s1[kBatch];
+    float m[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const int g = g0 + j;
+      if (g < G - 1) {
+        d[j] = st[static_cast<int64_t>(g) * kf4];
+        m[j] = exp2f(dec[g]);
+        s0[j] = pair < rot ? ph[g * 64] : 0.0;
+        s1[j] = pair + 1 < rot ? ph[g * 64 + 1] : 0.0;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (g0 + j < G - 1) {
+        float4 x = d[j];
+        if (pair < rot) {
+          float si, co;
+          sincospif(static_cast<float>(2.0 * (p0 - __builtin_rint(p0))), &si, &co);
+          x.x = d[j].x * co - d[j].y * si;
+          x.y = d[j].x * si + d[j].y * co;
+        }
+        if (pair + 1 < rot) {
+          float si, co;
+          sincospif(static_cast<float>(2.0 * (p1 - __builtin_rint(p1))), &si, &co);
+          x.z = d[j].z * co - d[j].w * si;
+          x.w = d[j].z * si + d[j].w * co;
+        }
+        p0 += s0[j], p1 += s1[j];
+        run.x = run.x * m[j] + x.x, run.y = run.y * m[j] + x.y;
+        run.z = run.z * m[j] + x.z, run.w = run.w * m[j] + x.w;
+        st[static_cast<int64_t>(g0 + j) * kf4] = run;
+      }
+    }
+  }
+}
+
+// Chunk-parallel plan, for fp32 operands (a summary's keys are rounded in its own
+// phase frame, which is the same state only while the rounding is the identity):
+// segments of at least two chunks, about one workgroup per CU.
+struct GenericPlan {
+  int G = 1;
+  int kf4 = 0, pt = 1;
+  int64_t decay_off = 0, phase_off = 0, bytes = 0;
+};
+
+bool rounds(const tf_mamba_args& a) {
+  return a.q_dtype != TF_FLOAT32 || a.k_dtype != TF_FLOAT32 || a.v_dtype != TF_FLOAT32;
+}
+
+GenericPlan generic_plan(const tf_mamba_args& a) {
+  GenericPlan p;
+  if (rounds(a) || !offsets_fit(a)) return p;
+  const int64_t units = a.batch * a.heads, chunks = (a.time + kChunk - 1) / kChunk;
+  if (units <= 0 || units > 128) return p;
+  const int64_t g = std::min<int64_t>(256 / units, chunks / 2);
+  if (g < 2) return p;
+  p.G = static_cast<int>(g);
+  const int nt = a.state <= 32 ? 1 : (a.state <= 64 ? 2 : 4);
+  p.pt = a.head_dim > 32 ? 2 : 1;
+  p.kf4 = nt * p.pt * 256;
+  auto up = [](int64_t x) { return (x + 255) & ~int64_t(255); };
+  p.phase_off = up(units * (g - 1) * p.kf4 * 16);
+  p.decay_off = p.phase_off + up(units * g * 64 * 8);
+  p.bytes = p.decay_off + up(units * g * 4);
+  return p;
 }
 
 template <typename I>
@@ -528,12 +697,32 @@ GenericParams<I> make_generic(const tf_mamba_args& a);
 
 template <int NT, int RP, typename I>
 int launch_pairs(const tf_mamba_args& a, hipStream_t stream) {
-  const GenericParams<I> P = make_generic<I>(a);
-  const dim3 grid(static_cast<uint32_t>(a.heads), static_cast<uint32_t>(a.batch));
-  if (a.q_dtype != TF_FLOAT32 || a.k_dtype != TF_FLOAT32 || a.v_dtype != TF_FLOAT32)
-    hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, true, I>), grid, dim3(kThreads), 0, stream, P);
-  else
-    hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, false, I>), grid, dim3(kThreads), 0, stream, P);
+  GenericParams<I> P = make_generic<I>(a);
+  const GenericPlan plan = generic_plan(a);
+  if (std::is_same_v<I, int32_t> && plan.G > 1 && a.workspace != nullptr && aligned(a.workspace, 256) &&
+      a.workspace_bytes >= plan.bytes) {
+    char* ws = static_cast<char*>(a.workspace);
+    P.G = plan.G;
+    P.state = reinterpret_cast<float4*>(ws);
+    P.phase = reinterpret_cast<double*>(ws + plan.phase_off);
+    P.decay = reinterpret_cast<float*>(ws + plan.decay_off);
+  }
+  const dim3 grid(static_cast<uint32_t>(a.heads), static_cast<uint32_t>(a.batch), static_cast<uint32_t>(P.G));
+  if (rounds(a)) {
+    hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, true, I, 0>), grid, dim3(kThreads), 0, stream, P);
+    return launch_status();
+  }
+  if constexpr (std::is_same_v<I, int32_t>) {
+    if (P.G > 1) {
+      hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, false, I, 1>), grid, dim3(kThreads), 0, stream, P);
+      if (const int rc = launch_status()) return rc;
+      const int64_t units = a.batch * a.heads;
+      hipLaunchKernelGGL(generic_scan_kernel<I>, dim3(static_cast<uint32_t>(units * (plan.kf4 / 64))), dim3(64), 0,
+                         stream, P, plan.kf4, plan.pt);
+      if (const int rc = launch_status()) return rc;
+    }
+  }
+  hipLaunchKernelGGL((mamba_generic_kernel<NT, RP, false, I, 0>), grid, dim3(kThreads), 0, stream, P);
   return launch_status();
 }
 
@@ -570,6 +759,10 @@ GenericParams<I> make_generic(const tf_mamba_args& a) {
   P.qvec = vec4(a.q, a.q_dtype, a.q_stride, a.state);
   P.kvec = vec4(a.k, a.k_dtype, a.k_stride, a.state);
   P.vvec = vec4(a.v, a.v_dtype, a.v_stride, a.head_dim);
+  P.G = 1;
+  P.state = nullptr;
+  P.decay = nullptr;
+  P.phase = nullptr;
   return P;
 }
 
@@ -577,6 +770,11 @@ GenericParams<I> make_generic(const tf_mamba_args& a) {
 
 bool generic_supported(const tf_mamba_args& a) {
   return a.state <= kNMax && a.head_dim <= kPMax;
+}
+
+int64_t generic_workspace_bytes(const tf_mamba_args& a) {
+  const GenericPlan plan = generic_plan(a);
+  return plan.G > 1 ? plan.bytes : 0;
 }
 
 int launch_generic(const tf_mamba_args& a, hipStream_t stream) {

@@ -17,6 +17,8 @@ __device__ __forceinline__ int valid_length(const tf_mamba_args& a, int b) {
 
 bool generic_supported(const tf_mamba_args& a);
 int launch_generic(const tf_mamba_args& a, hipStream_t stream);
+// Scratch bytes of its chunk-parallel form (fp32 operands; 0: one workgroup per unit).
+int64_t generic_workspace_bytes(const tf_mamba_args& a);
 
 bool mfma_supported(const tf_mamba_args& a);
 int launch_mfma(const tf_mamba_args& a, hipStream_t stream);
