@@ -131,6 +131,17 @@ int tf_fused_mamba(const tf_mamba_args *args, void *stream);
  */
 int64_t tf_fused_mamba_workspace_size(const tf_mamba_args *args);
 
+/*
+ * tf_fused_mamba with the generic kernel's chunk-parallel form as well (fp32
+ * operands): taken when args->workspace, 256-byte aligned, holds
+ * tf_fused_mamba_split_size(args) bytes, which tf_fused_mamba never asks for
+ * and never uses. Its sums are taken in another order, so results differ from
+ * tf_fused_mamba's in the last fp32 bits. For the other kernels both functions
+ * are tf_fused_mamba and tf_fused_mamba_workspace_size. No reference counterpart.
+ */
+int64_t tf_fused_mamba_split_size(const tf_mamba_args *args);
+int tf_fused_mamba_split(const tf_mamba_args *args, void *stream);
+
 /* Which kernel TF_MAMBA_AUTO would run for these arguments (1, 2 or 3), or a
  * negative tf_status if no kernel can run them. */
 int tf_fused_mamba_variant(const tf_mamba_args *args);

@@ -75,6 +75,12 @@ int select(const tf_mamba_args* a) {
   return -TF_ERR_SHAPE;
 }
 
+tf_mamba_args without_workspace(tf_mamba_args a) {
+  a.workspace = nullptr;
+  a.workspace_bytes = 0;
+  return a;
+}
+
 }  // namespace
 }  // namespace tf
 
@@ -86,7 +92,19 @@ extern "C" int tf_fused_mamba(const tf_mamba_args* a, void* stream) {
   if (tf::empty(a)) return TF_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (which == TF_MAMBA_PIPE) return tf::launch_pipe(*a, s);
-  return which == TF_MAMBA_MFMA ? tf::launch_mfma(*a, s) : tf::launch_generic(*a, s);
+  if (which == TF_MAMBA_MFMA) return tf::launch_mfma(*a, s);
+  return tf::launch_generic(tf::without_workspace(*a), s);
+}
+
+extern "C" int64_t tf_fused_mamba_split_size(const tf_mamba_args* a) {
+  const int which = tf::select(a);
+  if (which == TF_MAMBA_GENERIC && !tf::empty(a)) return tf::generic_workspace_bytes(*a);
+  return tf_fused_mamba_workspace_size(a);
+}
+
+extern "C" int tf_fused_mamba_split(const tf_mamba_args* a, void* stream) {
+  if (tf::select(a) == TF_MAMBA_GENERIC && !tf::empty(a)) return tf::launch_generic(*a, static_cast<hipStream_t>(stream));
+  return tf_fused_mamba(a, stream);
 }
 
 extern "C" int64_t tf_fused_mamba_workspace_size(const tf_mamba_args* a) {
@@ -94,7 +112,7 @@ extern "C" int64_t tf_fused_mamba_workspace_size(const tf_mamba_args* a) {
   if (which < 0) return which;
   if (tf::empty(a)) return 0;
   if (which == TF_MAMBA_PIPE) return tf::pipe_workspace_bytes(*a);
-  return which == TF_MAMBA_MFMA ? tf::mfma_workspace_bytes(*a) : tf::generic_workspace_bytes(*a);
+  return which == TF_MAMBA_MFMA ? tf::mfma_workspace_bytes(*a) : 0;
 }
 
 extern "C" int tf_fused_mamba_static(const tf_mamba_args* a, void* stream) {
@@ -102,18 +120,9 @@ extern "C" int tf_fused_mamba_static(const tf_mamba_args* a, void* stream) {
   if (which < 0) return -which;
   if (tf::empty(a)) return TF_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (which == TF_MAMBA_GENERIC) {
-    // its chunk-parallel form is not offered here: a long fp32 call's records
-    // would need more than the array holds, and the serial walk needs none
-    tf_mamba_args serial = *a;
-    serial.workspace = nullptr;
-    serial.workspace_bytes = 0;
-    return tf::launch_generic(serial, s);
-  }
+  if (which == TF_MAMBA_GENERIC) return tf::launch_generic(tf::without_workspace(*a), s);
   const int64_t need = which == TF_MAMBA_PIPE ? tf::pipe_workspace_bytes(*a) : tf::mfma_workspace_bytes(*a);
-  tf_mamba_args local = *a;
-  local.workspace = nullptr;
-  local.workspace_bytes = 0;
+  tf_mamba_args local = tf::without_workspace(*a);
   if (need > 0) {
     if (need > tf::kStaticScratchBytes) return TF_ERR_WORKSPACE;
     int device = -1;

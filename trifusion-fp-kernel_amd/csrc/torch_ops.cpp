@@ -132,7 +132,7 @@ at::Tensor& run(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
   // Long sequences over few (batch, head) units run chunk-parallel on scratch
   // the library sizes; it comes from torch's caching allocator on the current
   // stream (the graph's private pool under capture).
-  const int64_t need = tf_fused_mamba_workspace_size(&a);
+  const int64_t need = tf_fused_mamba_split_size(&a);
   if (need < 0) check_status(-need);
   at::Tensor workspace;
   if (need > 0) {
@@ -140,7 +140,7 @@ at::Tensor& run(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, c
     a.workspace = workspace.data_ptr();
     a.workspace_bytes = need;
   }
-  check_status(tf_fused_mamba(&a, c10::hip::getCurrentHIPStream(device.index()).stream()));
+  check_status(tf_fused_mamba_split(&a, c10::hip::getCurrentHIPStream(device.index()).stream()));
   return out;
 }
 

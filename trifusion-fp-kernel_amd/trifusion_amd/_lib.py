@@ -80,6 +80,8 @@ _SIGNATURES = {
     "tf_fused_mamba": ([ctypes.POINTER(MambaArgs), c_ptr], c_i32),
     "tf_fused_mamba_variant": ([ctypes.POINTER(MambaArgs)], c_i32),
     "tf_fused_mamba_workspace_size": ([ctypes.POINTER(MambaArgs)], c_i64),
+    "tf_fused_mamba_split": ([ctypes.POINTER(MambaArgs), c_ptr], c_i32),
+    "tf_fused_mamba_split_size": ([ctypes.POINTER(MambaArgs)], c_i64),
     "tf_fused_mamba_static": ([ctypes.POINTER(MambaArgs), c_ptr], c_i32),
     "tf_fused_mamba_static_scratch_bytes": ([], c_i64),
     "tf_rmsnorm": ([c_ptr, c_i32, c_i64, c_ptr, c_ptr, c_i32, c_i64, c_i64, c_f32, c_ptr], c_i32),
