@@ -588,6 +588,26 @@ int tf_grids(const int64_t *lengths, void *mask, int64_t *low_lengths, void *low
 int tf_log_spectrogram(const float *audio, const float *window, const int64_t *lengths, const int64_t *channels,
                        float *y, int64_t batch, int64_t chans, int64_t samples, void *stream);
 
+/*
+ * Bias-free linear layer whose output halves gate each other, x bf16 contiguous
+ * [rows, depth], w bf16 contiguous [2 features, depth], c = bf16(x w^T) with fp32
+ * sums, y bf16 contiguous [rows, features]:
+ *   kind 0: SwiGLU, y = bf16(silu(c[:, :features]) c[:, features:])  (swiglu after gate_up,
+ *           src/trifusion_l4/model.py:198)
+ *   kind 1: GLU, y = bf16(c[:, :features] sigmoid(c[:, features:]))  (F.glu after up, :73)
+ * features and depth multiples of 64, 16-byte aligned pointers.
+ */
+int tf_gated_linear(const void *x, const void *w, void *y, int64_t rows, int64_t features, int64_t depth,
+                    int32_t kind, void *stream);
+
+/*
+ * tf_glu_depthwise_norm_silu on rows that are gated already: x bf16 contiguous
+ * [B, T, D] in place of the [B, T, 2 D] rows it would gate.
+ */
+int tf_depthwise_norm_silu(const void *x, const void *w, const void *bias, const int64_t *lengths,
+                           const float *norm_w, float eps, void *y, int64_t batch, int64_t time, int64_t d,
+                           int64_t kernel, void *stream);
+
 /* Library version string (static storage). */
 const char *tf_version(void);
 

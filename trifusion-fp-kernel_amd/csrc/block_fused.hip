@@ -317,8 +317,10 @@ __global__ __launch_bounds__(256) void glu_depthwise_kernel(const uint16_t* __re
 // convolves output rows t0 + TO w .. + TO - 1 for every channel (lane = channel
 // groups 8 (lane + 64 j)), rounds them to bf16 as glu_depthwise's output is, and
 // normalises each row as norm_silu does (same per-lane order of the sum of
-// squares), so the values are those of the two launches.
-template <int K, int TW, int PER8>
+// squares), so the values are those of the two launches. GATED: the input rows
+// are gated already ([B, T, d], by the layer that formed them), so no row is
+// gated again for each tile whose halo it lies in (2.5 times at TW 4, K 7).
+template <int K, int TW, int PER8, bool GATED>
 __global__ __launch_bounds__(256) void glu_norm_silu_kernel(const uint16_t* __restrict__ up,
                                                             const uint16_t* __restrict__ w,
                                                             const uint16_t* __restrict__ bias,
@@ -344,9 +346,9 @@ __global__ __launch_bounds__(256) void glu_norm_silu_kernel(const uint16_t* __re
     const int idx = static_cast<int>(threadIdx.x) + 256 * i;
     const int r = idx / d8, c8 = idx < R * d8 ? idx - r * d8 : 0;
     const int t = min(max(t0 - K / 2 + r, 0), T - 1);
-    const uint16_t* src = up + (static_cast<int64_t>(b) * T + t) * 2 * d + 8 * c8;
+    const uint16_t* src = up + (static_cast<int64_t>(b) * T + t) * (GATED ? 1 : 2) * d + 8 * c8;
     ra[i] = *reinterpret_cast<const uint4*>(src);
-    rg[i] = *reinterpret_cast<const uint4*>(src + d);
+    if constexpr (!GATED) rg[i] = *reinterpret_cast<const uint4*>(src + d);
   }
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
@@ -354,6 +356,10 @@ __global__ __launch_bounds__(256) void glu_norm_silu_kernel(const uint16_t* __re
     if (idx < R * d8) {
       const int r = idx / d8, c8 = idx - r * d8;
       const int t = t0 - K / 2 + r;
+      if constexpr (GATED) {
+        glu_s[r * d8 + c8] = t >= 0 && t < T ? ra[i] : make_uint4(0u, 0u, 0u, 0u);
+        continue;
+      }
       float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       if (t >= 0 && t < T) {
         float a[8], g[8];
@@ -676,29 +682,48 @@ extern "C" int tf_norm_silu(const void* x, const float* w, void* y, int64_t rows
 #undef TF_NS
 }
 
-extern "C" int tf_glu_depthwise_norm_silu(const void* up, const void* w, const void* bias, const int64_t* lengths,
-                                          const float* norm_w, float eps, void* y, int64_t batch, int64_t time,
-                                          int64_t d, int64_t k, void* stream) {
+namespace tf {
+namespace {
+
+template <bool GATED>
+int launch_glu_norm_silu(const void* up, const void* w, const void* bias, const int64_t* lengths, const float* norm_w,
+                         float eps, void* y, int64_t batch, int64_t time, int64_t d, int64_t k, hipStream_t s) {
   if (!up || !w || !bias || !lengths || !norm_w || !y) return TF_ERR_NULL;
   if (batch < 0 || time < 0 || d < 8 || d % 8 || d > 1024 || batch > 65535 || batch * time > 0x7fffffff ||
-      (time + tf::kGnsTW - 1) / tf::kGnsTW > 65535)
+      (time + kGnsTW - 1) / kGnsTW > 65535)
     return TF_ERR_SHAPE;
-  if (!tf::a16(up) || !tf::a16(y) || !tf::a16(w) || !tf::a16(bias) || !tf::a16(norm_w)) return TF_ERR_SHAPE;
+  if (!a16(up) || !a16(y) || !a16(w) || !a16(bias) || !a16(norm_w)) return TF_ERR_SHAPE;
   if (batch * time == 0) return TF_OK;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(static_cast<uint32_t>((time + tf::kGnsTW - 1) / tf::kGnsTW), static_cast<uint32_t>(batch));
-  const size_t lds = static_cast<size_t>(tf::kGnsTW + k - 1) * (d / 8) * 16;
+  const dim3 grid(static_cast<uint32_t>((time + kGnsTW - 1) / kGnsTW), static_cast<uint32_t>(batch));
+  const size_t lds = static_cast<size_t>(kGnsTW + k - 1) * (d / 8) * 16;
 #define TF_GNS(KV, P)                                                                                            \
   if (k == KV && (d <= 512 * P) && (P == 1 || d > 512 * (P / 2))) {                                              \
-    hipLaunchKernelGGL((tf::glu_norm_silu_kernel<KV, tf::kGnsTW, P>), grid, dim3(256), lds, s,                 \
+    hipLaunchKernelGGL((glu_norm_silu_kernel<KV, kGnsTW, P, GATED>), grid, dim3(256), lds, s,                    \
                        static_cast<const uint16_t*>(up), static_cast<const uint16_t*>(w),                        \
                        static_cast<const uint16_t*>(bias), lengths, norm_w, static_cast<uint16_t*>(y),          \
                        static_cast<int>(time), static_cast<int>(d), eps);                                        \
-    return tf::launch_status();                                                                                  \
+    return launch_status();                                                                                      \
   }
   TF_GNS(3, 1) TF_GNS(3, 2) TF_GNS(7, 1) TF_GNS(7, 2)
 #undef TF_GNS
   return TF_ERR_SHAPE;
+}
+
+}  // namespace
+}  // namespace tf
+
+extern "C" int tf_glu_depthwise_norm_silu(const void* up, const void* w, const void* bias, const int64_t* lengths,
+                                          const float* norm_w, float eps, void* y, int64_t batch, int64_t time,
+                                          int64_t d, int64_t k, void* stream) {
+  return tf::launch_glu_norm_silu<false>(up, w, bias, lengths, norm_w, eps, y, batch, time, d, k,
+                                         static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tf_depthwise_norm_silu(const void* x, const void* w, const void* bias, const int64_t* lengths,
+                                      const float* norm_w, float eps, void* y, int64_t batch, int64_t time, int64_t d,
+                                      int64_t k, void* stream) {
+  return tf::launch_glu_norm_silu<true>(x, w, bias, lengths, norm_w, eps, y, batch, time, d, k,
+                                        static_cast<hipStream_t>(stream));
 }
 
 extern "C" int tf_glu_depthwise(const void* up, const void* w, const void* bias, const int64_t* lengths, void* y,

@@ -145,6 +145,11 @@ _SIGNATURES = {
         [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_f32, c_ptr, c_i64, c_i64, c_i64, c_i64, c_ptr],
         c_i32,
     ),
+    "tf_depthwise_norm_silu": (
+        [c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_f32, c_ptr, c_i64, c_i64, c_i64, c_i64, c_ptr],
+        c_i32,
+    ),
+    "tf_gated_linear": ([c_ptr, c_ptr, c_ptr, c_i64, c_i64, c_i64, c_i32, c_ptr], c_i32),
     "tf_interpolate_rmsnorm": (
         [c_ptr, c_i32, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_f32, c_ptr, c_i64, c_i64, c_i64, c_i64, c_ptr],
         c_i32,

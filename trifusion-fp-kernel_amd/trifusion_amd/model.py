@@ -29,6 +29,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .kernels import RMSNorm, swiglu
+from .kernels.block import gated_linear, gated_linear_fits
 from .kernels.native import add, add_rms, mask_rms, mean_norm
 from .mamba import Mamba3Inference, weight_key
 from .masking import masked_mean
@@ -70,12 +71,12 @@ class EncoderBlock(nn.Module):
         self.down = nn.Linear(c.ffn_dim, c.dim, bias=False)
         self._padded = None
         self._padded_key = None
+        self._kmajor = None
 
-    def _padded_ffn(self):
-        """The FFN weights at a width the library GEMMs run well: each half of
-        gate_up zero-padded to a multiple of FFN_ALIGN rows and stored K-major
-        ([dim, 2 * width], used as ``h @ w``), and down with matching zero
-        columns. An odd width (1365) leaves every GEMM tile and SwiGLU row
+    def _padded_rows(self):
+        """The FFN weights at a width the GEMMs run well: each half of gate_up
+        zero-padded to a multiple of FFN_ALIGN rows ([2 * width, dim]), and
+        down with matching zero columns. An odd width (1365) leaves every GEMM tile and SwiGLU row
         misaligned; the padded rows give silu(0) * 0 = 0 and meet zero columns
         of down, so the result is the same up to the GEMMs' summation order.
         Rebuilt when either weight changes."""
@@ -90,10 +91,22 @@ class EncoderBlock(nn.Module):
                 g1[fp : fp + f] = w1[f:]
                 g2 = w2.new_zeros(d, fp)
                 g2[:, :f] = w2
-            self._padded, self._padded_key = (g1.t().contiguous(), g2), key
+            self._padded, self._padded_key = (g1, g2), key
         return self._padded
 
+    def _padded_ffn(self):
+        """``_padded_rows`` with gate_up stored K-major ([dim, 2 * width], used
+        as ``h @ w``), as the library GEMM runs it best."""
+        g1, g2 = self._padded_rows()
+        hit = self._kmajor
+        if hit is None or hit[1] is not g2:
+            hit = self._kmajor = (g1.t().contiguous(), g2)
+        return hit
+
     def ffn(self, h):
+        g1, g2 = self._padded_rows()
+        if gated_linear_fits(h, g1):
+            return F.linear(gated_linear(h, g1, "swiglu"), g2)
         g1t, g2 = self._padded_ffn()
         return F.linear(swiglu(h @ g1t), g2)
 

@@ -86,6 +86,11 @@ _SCHEMAS = {
     "glu_norm_silu": (
         "glu_norm_silu(Tensor up, Tensor weight, Tensor bias, Tensor lengths, Tensor norm_weight, float eps) -> Tensor"
     ),
+    "depthwise_norm_silu": (
+        "depthwise_norm_silu(Tensor x, Tensor weight, Tensor bias, Tensor lengths, Tensor norm_weight, float eps) "
+        "-> Tensor"
+    ),
+    "gated_linear": "gated_linear(Tensor x, Tensor weight, str kind) -> Tensor",
     "merge_conv": (
         "merge_conv(Tensor cn, Tensor mn, Tensor an, Tensor g, Tensor weight, Tensor bias, Tensor lengths) -> Tensor"
     ),
@@ -348,6 +353,14 @@ def _meta_glu_norm_silu(up, weight, bias, lengths, norm_weight, eps):
     return up.new_empty((*up.shape[:-1], up.shape[-1] // 2), dtype=torch.bfloat16)
 
 
+def _meta_depthwise_norm_silu(x, weight, bias, lengths, norm_weight, eps):
+    return torch.empty_like(x, memory_format=torch.contiguous_format)
+
+
+def _meta_gated_linear(x, weight, kind):
+    return x.new_empty((*x.shape[:-1], weight.shape[0] // 2))
+
+
 def _meta_evidence_down(cn, an, weight, bias):
     return cn.new_empty((*cn.shape[:-1], weight.shape[0]), dtype=torch.bfloat16)
 
@@ -446,8 +459,8 @@ _KERNELS = {
         name: (_block(name), globals()["_meta_" + name])
         for name in ("depthwise_masked", "pool4", "rotary_qkv", "front_norm", "interpolate", "interpolate_rmsnorm",
                      "bands", "evidence_norm", "gated_concat", "front_conv1", "front_conv2", "block_pre",
-                     "block_pre_add", "norm_silu", "glu_depthwise", "glu_norm_silu", "pooled_attention", "merge_gate",
-                     "evidence_down", "merge_conv", "query_read", "mask_audio", "log_power", "log_spectrogram",
+                     "block_pre_add", "norm_silu", "glu_depthwise", "glu_norm_silu", "depthwise_norm_silu", "gated_linear",
+                     "pooled_attention", "merge_gate", "evidence_down", "merge_conv", "query_read", "mask_audio", "log_power", "log_spectrogram",
                      "front_lengths", "grids")
     },
 }

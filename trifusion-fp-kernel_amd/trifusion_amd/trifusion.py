@@ -42,11 +42,15 @@ from .kernels.block import (
     block_pre_add,
     block_pre_add_fits,
     depthwise_masked,
+    depthwise_norm_silu,
+    depthwise_norm_silu_fits,
     evidence_down,
     evidence_down_fits,
     evidence_norm,
     front_norm,
     front_stage,
+    gated_linear,
+    gated_linear_fits,
     glu_depthwise,
     glu_norm_silu,
     glu_norm_silu_fits,
@@ -255,6 +259,14 @@ class Frontend(nn.Module):
         return bands(x).flatten(2), fine, lengths, fine_lengths
 
 
+def _gates(layer, x):
+    """Whether ``layer(x)`` and the gate after it run as one ``gated_linear``: a
+    plain bias-free layer (no subclass, hook or replaced forward that the
+    fused call would pass by) on operands the kernel takes."""
+    return (type(layer) is nn.Linear and layer.bias is None and not layer._forward_pre_hooks
+            and not layer._forward_hooks and "forward" not in vars(layer) and gated_linear_fits(x, layer.weight))
+
+
 class LocalCNN(nn.Module):
     """GLU -> masked depthwise conv (7) -> RMSNorm -> SiLU -> linear (``model.py:51-75``)."""
 
@@ -373,6 +385,9 @@ class TriFusionBlock(nn.Module):
         """GLU, masked depthwise conv, norm, SiLU, out-projection and the cn
         norm: ``cn``."""
         local = self.local
+        if _gates(local.up, h) and depthwise_norm_silu_fits(h.shape[-1], local.dw):
+            up = gated_linear(h, local.up.weight, "glu")
+            return self.cn(local.out(depthwise_norm_silu(up, local.dw, lengths, local.norm)))
         up = local.up(h)
         if glu_norm_silu_fits(up, local.dw):
             return self.cn(local.out(glu_norm_silu(up, local.dw, lengths, local.norm)))
@@ -444,7 +459,7 @@ class TriFusionBlock(nn.Module):
         mn, g = merge_gate(cn, mf, mb, an, self.mn, self.gate)
         merged = self.merge(merge_conv(cn, mn, an, g, self.merge_dw, lengths))
         r, f = add_rms(x, merged, self.ff_norm.weight, None, self.ff_norm.eps, torch.bfloat16)
-        f = swiglu(self.gate_up(f))
+        f = gated_linear(f, self.gate_up.weight, "swiglu") if _gates(self.gate_up, f) else swiglu(self.gate_up(f))
         down = self.down(f)
         if defer and down.dtype == torch.bfloat16 and block_pre_add_fits(r, down):
             return (r, down), mf, mb
