@@ -14,10 +14,11 @@ DEV = "cuda:0"
 
 @pytest.mark.parametrize(
     "rows,features,depth",
-    # 64-row tiles: one to three stages, a partial tile, nine row tiles; 128-row
-    # tiles (from 257 of them on): exact, one row over, a partial last group
-    [(1, 64, 64), (63, 64, 128), (65, 128, 192), (129, 192, 256), (523, 64, 64), (128 * 17, 1024, 64),
-     (128 * 16 + 1, 1024, 128), (128 * 22 - 3, 768, 192)],
+    # 64-row tiles: one to three stages, a partial tile, nine row tiles; then tiles of
+    # 160 (2049, 2176, 4223 rows), 192 (1801, 1920) and 128 rows (3969, 4096): exact,
+    # one row over, a partial last group
+    [(1, 64, 64), (63, 64, 128), (65, 128, 192), (129, 192, 256), (523, 64, 64), (2049, 1024, 128), (2176, 1024, 64),
+     (4223, 1024, 192), (1801, 2816, 64), (1920, 1408, 64), (3969, 1024, 64), (4096, 1024, 128)],
 )
 @pytest.mark.parametrize("kind", ["swiglu", "glu"])
 def test_against_float64(rows, features, depth, kind):

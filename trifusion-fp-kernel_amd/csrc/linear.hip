@@ -6,20 +6,22 @@
 // each half, rounded to bf16 in LDS as the separate product's output is, and the
 // gate runs on those values with the separate kernels' arithmetic.
 //
-// A tile is BM rows by 64 + 64 columns, four waves (two by two) on MFMA 32x32x16.
+// A tile is BM rows by 64 + 64 columns, four waves (WR by 4 / WR) on MFMA 32x32x16.
 // Operands go straight from memory into LDS (16 bytes per lane, no registers),
 // 64 of K per stage, S stages deep; a stage's rows are 128 bytes and the lane that
 // fetches slot p of row r takes piece p ^ (r % 8), so that the operand reads (32
 // rows, one piece) fall on distinct banks. Two workgroups share a CU.
 //
 // What bounds it: the way from L2 into a CU, ~100 KB/us per CU here (26 TB/s over
-// the chip), which a 128 x 128 tile asks 32 KB of for every 64 of K; so the larger
-// tile is taken where it has work for every CU, and the 64-row tile (three stages,
-// twice the workgroups) below that. SwiGLU layer, against the library's product and
-// a gate kernel: 6400 x (2 x 1408) x 512 41.2 -> 29.0 us, 1616 x (2 x 2816) x 1024
-// 36.0 -> 29.3, 404 rows 17.5 -> 11.3, 28 816 rows 364 -> 349; one row of 64 6.1 ->
-// 2.9. GLU, 1616 x (2 x 1024) x 1024: 13.2 us against 12.3 for the library's product
+// the chip), which a tile asks (BM + 128) x 128 bytes of for every 64 of K; so the
+// rows of a tile are chosen for the least of that on the busiest CU (see the launch),
+// and the 64-row tile (three stages) is for grids that do not fill the chip. SwiGLU
+// layer, against the library's product and a gate kernel: 6400 x (2 x 1408) x 512
+// 41.2 -> 25.8 us, 1616 x (2 x 2816) x 1024 36.0 -> 27.3, 404 rows 17.5 -> 11.3,
+// 28 816 rows 364 -> 334; one row of 64 6.1 -> 2.9. GLU, 1616 x (2 x 1024) x 1024: 13.2 us against 12.3 for the library's product
 // alone, and the convolution after it 12.4 -> 8.0 on rows that are gated once.
+#include <algorithm>
+
 #include "mfma_tile.h"
 
 namespace tf {
@@ -59,10 +61,10 @@ __device__ __forceinline__ void stage_barrier() {
 __device__ __forceinline__ float glu(float a, float g) { return a * (1.0f / (1.0f + expf(-g))); }
 __device__ __forceinline__ float swiglu(float g, float u) { return g * sigmoidf(g) * u; }
 
-template <int BM, int S, bool SWIGLU>
+template <int BM, int S, int WR, bool SWIGLU>
 __global__ __launch_bounds__(kThreads) void gated_linear_kernel(const GatedArgs P) {
   constexpr int FPW = (BM + kBN) / 8 / 4;  // fetches per wave and stage, 8 rows each
-  constexpr int MT = BM / 64, NT = 2;      // 32 x 32 tiles per wave
+  constexpr int WC = 4 / WR, MT = BM / 32 / WR, NT = 4 / WC;  // 32 x 32 tiles per wave
   constexpr int STAGE = (BM + kBN) * kStep;
   static_assert(S * STAGE >= BM * kCS, "the output tile takes the stages' memory");
   __shared__ __align__(1024) uint16_t lds[S * STAGE];
@@ -99,8 +101,8 @@ __global__ __launch_bounds__(kThreads) void gated_linear_kernel(const GatedArgs 
 #pragma unroll
     for (int i = 0; i < FPW; ++i) fetch(to + 1024u * i, off[i], 8 * (w * FPW + i) < BM ? xk : wk);
   };
-  const int wr = w >> 1, wc = w & 1;
-  const int xr = (wr * (BM / 2) + c32) * kStep, wro = (BM + wc * kHalf + c32) * kStep, swz = c32 & 7;
+  const int wr = w / WC, wc = w % WC;
+  const int xr = (wr * (BM / WR) + c32) * kStep, wro = (BM + wc * (kBN / WC) + c32) * kStep, swz = c32 & 7;
   f32x16 acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -153,7 +155,8 @@ __global__ __launch_bounds__(kThreads) void gated_linear_kernel(const GatedArgs 
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<u32x2*>(lds + (wr * (BM / 2) + 32 * i + c32) * kCS + wc * kHalf + 32 * j + 8 * g + 4 * hh) =
+        *reinterpret_cast<u32x2*>(lds + (wr * (BM / WR) + 32 * i + c32) * kCS + wc * (kBN / WC) + 32 * j + 8 * g +
+                                  4 * hh) =
             u32x2{pack2(acc[i][j][4 * g], acc[i][j][4 * g + 1]), pack2(acc[i][j][4 * g + 2], acc[i][j][4 * g + 3])};
   __syncthreads();
 #pragma unroll
@@ -172,15 +175,15 @@ __global__ __launch_bounds__(kThreads) void gated_linear_kernel(const GatedArgs 
   }
 }
 
-template <int BM, int S>
+template <int BM, int S, int WR>
 int launch_gated(GatedArgs P, bool swiglu, hipStream_t s) {
   P.tm = (P.M + BM - 1) / BM;
   P.tn = P.F / kHalf;
   const dim3 grid(static_cast<uint32_t>(P.tm) * P.tn), block(kThreads);
   if (swiglu)
-    hipLaunchKernelGGL((gated_linear_kernel<BM, S, true>), grid, block, 0, s, P);
+    hipLaunchKernelGGL((gated_linear_kernel<BM, S, WR, true>), grid, block, 0, s, P);
   else
-    hipLaunchKernelGGL((gated_linear_kernel<BM, S, false>), grid, block, 0, s, P);
+    hipLaunchKernelGGL((gated_linear_kernel<BM, S, WR, false>), grid, block, 0, s, P);
   return launch_status();
 }
 
@@ -204,10 +207,20 @@ extern "C" int tf_gated_linear(const void* x, const void* w, void* y, int64_t ro
   tf::GatedArgs P{static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), static_cast<uint16_t*>(y),
                   static_cast<int>(rows), static_cast<int>(features), static_cast<int>(depth), 0, 0};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // 128-row tiles from more than one per CU on (256 CUs). 1024 x 1024, K 1024: 128
-  // tiles 12.4 us against 9.3 in 64-row tiles, 256 tiles 13.1 against 12.3, 400
-  // tiles 18.1 against 21.9; 2816 features: 220 tiles 12.8 against 12.9, 264 tiles
-  // 16.7 against 18.6, 704 tiles 29.1 against 33.9
-  if ((rows + 127) / 128 * (features / tf::kHalf) > 256) return tf::launch_gated<128, 2>(P, kind == 0, s);
-  return tf::launch_gated<64, 3>(P, kind == 0, s);
+  // 64-row tiles up to one 128-row tile per CU (256 CUs). K 1024, 1024 features: 128
+  // tiles 9.3 us against 12.4 in 128-row tiles, 256 tiles 12.3 against 13.1, 400
+  // tiles 21.9 against 18.1; 2816 features: 220 tiles 12.9 against 12.8, 264 tiles
+  // 18.6 against 16.7.
+  const int64_t cols = features / tf::kHalf;
+  const auto tiles = [&](int64_t bm) { return (rows + bm - 1) / bm * cols; };
+  if (tiles(128) <= 256) return tf::launch_gated<64, 3, 2>(P, kind == 0, s);
+  // Above that the tile whose busiest CU fetches least, which orders what the tiles
+  // take (us, 128 / 160 / 192 rows): 1616 x 2816, K 1024 29.5 / 24.9 / 24.7, 1801
+  // rows 28.6 / 36.6 / 26.3, 28 816 rows 340 / 356 / 322; 6400 x 1408, K 512 27.6 /
+  // 26.8 / 24.7, 1608 rows 11.5 / 10.7 / 11.3.
+  const auto cost = [&](int64_t bm) { return (tiles(bm) + 255) / 256 * (bm + tf::kBN); };
+  const int64_t best = std::min({cost(128), cost(160), cost(192)});
+  if (cost(128) == best) return tf::launch_gated<128, 2, 2>(P, kind == 0, s);
+  if (cost(160) == best) return tf::launch_gated<160, 2, 1>(P, kind == 0, s);
+  return tf::launch_gated<192, 2, 2>(P, kind == 0, s);
 }
