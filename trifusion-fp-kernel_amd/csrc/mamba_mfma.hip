@@ -263,10 +263,6 @@ __global__ __launch_bounds__(CW * 128) void mamba_mfma_kernel(const MfmaParams P
   // loading its rows after phase pass 1, which staggers the two halves' bursts;
   // prefetching both halves, or issuing the next controls before the scan, was
   // slower.
-  // N = 128, P = 64 with one chunk per super-chunk runs at one wave per SIMD
-  // and spills into AGPRs; the next chunk's rows are loaded where used instead
-  // of being held across the chunk.
-  constexpr bool kPrefetch = !(NT == 4 && PT == 2 && CW == 1);
   HalfRows<KS, PS> pre = {};
   for (int g0 = c_begin; g0 < c_stop; g0 += CW) {
     // Lane-derived indices are rebuilt from an index the compiler cannot see
@@ -294,7 +290,7 @@ __global__ __launch_bounds__(CW * 128) void mamba_mfma_kernel(const MfmaParams P
     // wave of each SIMD computes while the other waits.
     HalfRows<KS, PS> rows = {};
     if (active && hf == 0) {
-      if (g0 == c_begin || !kPrefetch)
+      if (g0 == c_begin)
         load_rows<MODE == 0>(P, rows, qbase, kbase, vbase, t0, t, L, hh);
       else
         rows = pre;
@@ -596,7 +592,7 @@ __global__ __launch_bounds__(CW * 128) void mamba_mfma_kernel(const MfmaParams P
     }
     lds_barrier();  // barrier 3: every dS share in LDS
     pre = {};
-    if (kPrefetch && hf == 0 && g0 + CW + cw < c_stop) {
+    if (hf == 0 && g0 + CW + cw < c_stop) {
       const int t0n = (g0 + CW + cw) * kChunk;
       load_rows<MODE == 0>(P, pre, qbase, kbase, vbase, t0n, t0n + c32, L, hh);
     }
@@ -991,12 +987,11 @@ bool mfma_supported(const tf_mamba_args& a) {
   return offsets_fit(a);
 }
 
-// Four chunks (eight waves, two per SIMD) per super-chunk. N=128 keeps two
+// Four chunks (eight waves, two per SIMD) per super-chunk. N=128, P=32 keeps two
 // chunks (four waves, one per SIMD): its working set needs the 512 registers a
-// lone wave gets, and with P=64 its two LDS slots per chunk would not fit four.
-// With more (batch, head) units than CUs, N=128, P=64 takes one chunk per
-// super-chunk: its 69 KB of LDS lets two workgroups share a CU, so every unit
-// runs in one round instead of two (the model's 16 x 32 units: 37.8 -> 34.2 us).
+// lone wave gets. N=128, P=64 runs on mamba_wide.hip at every size: 512 units of
+// 101 rows took 38.6 us here and take 21.0 there, 32 units of 1801 rows 92.3 and
+// 49.9.
 int launch_mfma(const tf_mamba_args& a, hipStream_t stream) {
   const int nt = static_cast<int>(padded_state(a) / 32);
   const int pt = static_cast<int>(a.head_dim / 32);

@@ -25,6 +25,13 @@
 // holds index 32 s + 16 (j / 4) + 4 g + j % 4, which is where a pair of D tiles
 // holds its rows.
 //
+// What bounds it: vector instructions (about 2300 per wave and chunk, rotation and
+// controls before all; the matrix cores are busy for a tenth of that) and, on short
+// walks, the first chunk's loads and controls (a quarter of the time at 101 rows).
+// Measured, bf16 projections, H = 32, one direction, the chunked kernel of
+// mamba_mfma.hip against this one (us): 16 x 101 rows 38.6, 21.0; 8 x 201 41.4, 27.6;
+// 4 x 401 90.8, 47.2; 1 x 1801 92.3, 49.9.
+//
 // Chunk-parallel form (few long units): summaries of every segment but the last
 // (this kernel, MODE 1: from zero state and phase, only keys and values), a scan
 // that turns each summary into the state entering the next segment, and the
@@ -621,9 +628,15 @@ __global__ __launch_bounds__(64) void wide_scan_kernel(const MfmaParams P) {
   }
 }
 
-// Chunk-parallel plan: segments of at least kMinChunks chunks, about kGroups
-// workgroups, and records that fit the library's static scratch.
-constexpr int64_t kGroups = 512, kMinChunks = 2, kMaxUnits = 128, kMaxRecords = 480;
+// Chunk-parallel plan. At most kGroups workgroups (two on each of the 256 CUs, all
+// resident) and records that fit the library's static scratch (kMaxRecords of
+// 32 KB, and the phases, in 16 MiB); segments as short as that allows, but of two
+// chunks. The summaries, the scan and their launches pay from six chunks on, from
+// eight above 96 units, and up to 170 units, which leave three segments each (us,
+// split against serial): 64 units, 4 chunks 29.7 / 26.8, 5 40.3 / 34.4, 6 32.2 / 40.8,
+// 29 70.8 / 193; 128 units, 7 chunks 46.3 / 47.0, 8 45.8 / 55.6; 160 units, 7 chunks
+// 51.4 / 48.3, 13 74.3 / 89.6; 192 units in two segments, 13 chunks 96.5 / 89.6.
+constexpr int64_t kGroups = 512, kMaxRecords = 480, kSegment = 2, kMaxUnits = 170;
 
 struct WidePlan {
   int G = 1;
@@ -636,9 +649,8 @@ WidePlan wide_plan(const tf_mamba_args& a) {
   WidePlan p;
   const int64_t units = a.batch * a.heads;
   const int64_t chunks = (a.time + kChunk - 1) / kChunk;
-  if (units <= 0 || units > kMaxUnits) return p;
-  const int64_t g = std::min({kGroups / units, chunks / kMinChunks, kMaxRecords / units + 1});
-  if (g < 2) return p;
+  if (units <= 0 || units > kMaxUnits || chunks < (units <= 96 ? 6 : 8)) return p;
+  const int64_t g = std::min({kGroups / units, kMaxRecords / units + 1, (chunks + kSegment - 1) / kSegment});
   p.G = static_cast<int>(g);
   auto up = [](int64_t x) { return (x + 255) & ~int64_t(255); };
   p.phase_off = up(units * (g - 1) * kRecF4 * 16);

@@ -69,7 +69,7 @@ class Mamba3Inference(nn.Module):
         self.D = nn.Parameter(torch.ones(self.nheads))
         self.B_norm = RMSNorm(self.d_state)
         self.C_norm = RMSNorm(self.d_state)
-        # "pipe" (pipelined MFMA walk), "mfma" (chunked MFMA scan), "generic" (fp32-FMA kernel) or "auto"
+        # "pipe" (pipelined MFMA walk), "mfma" (chunked MFMA scan), "generic" (fp32 MFMA kernel) or "auto"
         self.variant = "auto"
         self.fuse_controls = True
         self.fuse_norms = True

@@ -7,7 +7,7 @@ Same API and policies as the reference runtime (``src/trifusion_l4/runtime.py``)
     with ``torch.load(weights_only=True, mmap=True)``, rejects unknown config
     keys, builds the model on the meta device, attaches the tensors with
     ``load_state_dict(strict=True, assign=True)``, freezes it and casts the GEMM
-    weights to bf16. ``optimized=False`` selects the generic (fp32-FMA) recurrence
+    weights to bf16. ``optimized=False`` selects the generic (fp32 MFMA) recurrence
     kernel instead of the MFMA chunked scan.
 ``configure_runtime(threads=2, enforce_gfx950=True)`` (``:57-65``)
     Requires a ROCm GPU, by default a gfx950 (MI355X) one, sets the host thread
