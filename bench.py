@@ -57,7 +57,7 @@ COUNTERS_FILE = ROOT / "profiles" / "fused_mamba_clip_b16_l400_counters.txt"
 # these it was measured on, and its figures are reported only if it matches
 KERNEL_SOURCES = [
     ROOT / "trifusion-fp-kernel_amd" / "csrc" / name
-    for name in ("mamba_pipe.hip", "mfma_tile.h", "mamba_internal.h", "common.h")
+    for name in ("mamba_pipe.hip", "mamba_walk.h", "mfma_tile.h", "mamba_internal.h", "common.h")
 ]
 
 

@@ -1,5 +1,5 @@
 // Matrix-core tile helpers and the kernel-side operand block shared by the
-// gfx950 recurrence kernels (mamba_mfma.hip, mamba_pipe.hip).
+// gfx950 recurrence, attention and linear kernels.
 //
 // MFMA 32x32x16 register layout (lane l, c32 = l & 31, hh = l >> 5):
 //   A[i][k]: lane i + 32*(k/8), element k%8
