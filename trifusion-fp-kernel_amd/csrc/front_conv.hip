@@ -49,11 +49,18 @@ __device__ __forceinline__ int clamp_len(const int64_t* lengths, int b, int T) {
   return l < 0 ? 0 : (l > T ? T : static_cast<int>(l));
 }
 
-// SiLU in fp32, y / (1 + e^-y), from the hardware exp2 and reciprocal (each within
-// about 1 ulp); its result is rounded to bf16. The epilogues run it once per
-// output value: with expf and an IEEE division it was a third of a stage's time.
+// SiLU of a bf16 value, y / (1 + e^-y), rounded to bf16 by the caller. The hardware
+// exp2 of a rounded argument is off by more as |y| grows (50 units of fp32 at 80) and
+// the hardware reciprocal by one, less a Newton step; what counts is the bf16 result,
+// which is the correctly rounded one for every bf16 y down to -87 (without the Newton
+// step all but 5.9375, a value the norm of a lone large channel gives often). Below
+// that the reciprocal is 0, and the maximum takes the step's 0 x infinity away. With
+// expf and an IEEE division, the same results, the epilogues, which run it once per
+// output value, were a third of a stage's time.
 __device__ __forceinline__ float silu(float y) {
-  return y * __builtin_amdgcn_rcpf(1.0f + fast_exp2(-y * 1.4426950408889634f));
+  const float d = 1.f + fast_exp2(-y * 1.4426950408889634f);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return y * __builtin_fmaf(fmaxf(__builtin_fmaf(-d, r, 1.f), -1.f), r, r);
 }
 
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
