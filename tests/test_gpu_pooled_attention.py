@@ -98,3 +98,29 @@ def test_query_read_merges_many_tiles(t, lengths):
     # half a bf16 step and fp32 sums of values up to ~5
     assert (err <= ref.abs()[some] * 2.0**-8 + 5 * 64 * 2.0**-23).all(), err.max()
     assert not y[~some].any()
+
+
+def test_small_probabilities_are_rounded_once():
+    """Two keys, scores 0 and -x for x in 40..70, values 0 and 1: the output is
+    e^-x / (1 + e^-x), in bf16. The score, the sum and the reciprocal are exact, so
+    what stands between it and the correctly rounded value is the exponential. One
+    that is off by a unit of 2^-23 everywhere would turn one result in 2^15 (twice the
+    error over the least step of a bf16 mantissa, 2^-7): 2 to 3 of 65 536, and 4 are
+    allowed. One whose argument is a rounded product turned 16."""
+    t, heads, hd = 4096, 16, 64
+    g = torch.Generator().manual_seed(8)
+    # x = (a b + c) / 8 in multiples of 2^-12
+    a, b = (torch.rand(t, heads, generator=g) * 4 + 16).to(BF), (torch.rand(heads, generator=g) * 6 + 21).to(BF)
+    c = (torch.rand(t, heads, generator=g) / 2 + 0.5).to(BF)
+    qkv = torch.zeros(1, t, 3, heads, hd, dtype=BF)
+    qkv[0, :, 0, :, 0], qkv[0, :, 0, :, 2] = a, c
+    qkv[0, 1, 1, :, 0], qkv[0, 1, 1, :, 2] = -b, -1
+    qkv[0, 1, 2, :, 0] = 1
+    cos, sin = torch.ones(t, hd // 2), torch.zeros(t, hd // 2)
+    grids = SimpleNamespace(rope_cos=cos.to(DEV), rope_sin=sin.to(DEV), low_lengths=torch.tensor([2], device=DEV))
+    y = pooled_attention(qkv.reshape(1, t, -1).to(DEV), grids, heads).cpu().view(t, heads, hd)[..., 0]
+    x = (a.double() * b.double() + c.double()) / 8
+    ref = (1 / (1 + x.exp())).float().to(BF)
+    differ = int((y != ref).sum())
+    print(f"{differ} of {y.numel()} results not the correctly rounded ones", flush=True)
+    assert differ <= 4

@@ -21,9 +21,11 @@
 // softmax, six or twelve products), since a bucket of files has few tiles: at
 // most 256 workgroups for 16 clips of 26 pooled rows or one file of 451. A kernel
 // that formed the dot products on the vector units, four lanes to a query, and
-// walked all keys in one wave took 11.2 us at 16 clips of 26 pooled rows, 31.0 at
-// 4 of 101 and 123.7 at one file of 451 (16 heads of 64; graph-replayed); this one
-// takes 4.8, 7.3 and 13.5, with the same distance from a float64 evaluation.
+// walked all keys in one wave took 11.8 us at 16 clips of 26 pooled rows, 32.0 at
+// 4 of 101 and 123 at one file of 451 (16 heads of 64; calls of a graph, end to
+// end); this one takes 5.9, 9.0 and 15.8, with the same distance from a float64
+// evaluation. A tenth of that is expf: the hardware exp2 of a rounded product takes
+// 5.5, 8.1 and 14.4, and is 20 units of fp32 off where the difference is 50.
 #include "mfma_tile.h"
 
 namespace tf {
@@ -98,8 +100,6 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(const uint16_t* __re
   const uint16_t* base = qkv + static_cast<int64_t>(b) * LT * width + static_cast<int64_t>(h) * D;
   const uint16_t* kbase = base + static_cast<int64_t>(H) * D;
   const uint16_t* vbase = base + static_cast<int64_t>(2) * H * D;
-  // exp(scale (s - m)) = 2^((s - m) c)
-  const float c = scale * 1.4426950408889634f;
 
   // row `t`, as the MFMA operand whose lane (c32, hh) holds dims 16 s + 8 hh + j
   auto rotated = [&](const uint16_t* rows, int t, u32x4 (&out)[KS]) {
@@ -151,17 +151,19 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(const uint16_t* __re
     f32x16 s = zero16();
 #pragma unroll
     for (int i = 0; i < KS; ++i) s = mfma(k[i], q[i], s);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] *= scale;
     // online softmax of query c32 over keys j0 + drow(e, hh)
     float mx = m;
 #pragma unroll
     for (int e = 0; e < 16; ++e) mx = fmaxf(mx, drow(e, hh) < nk ? s[e] : -INFINITY);
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float corr = m == mx ? 1.f : fast_exp2((m - mx) * c);
+    const float corr = m == mx ? 1.f : expf(m - mx);
     float p[16];
     float sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      p[e] = drow(e, hh) < nk ? fast_exp2((s[e] - mx) * c) : 0.f;
+      p[e] = drow(e, hh) < nk ? expf(s[e] - mx) : 0.f;
       sum += p[e];
     }
     sum += __shfl_xor(sum, 32, 64);
@@ -242,7 +244,7 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(const uint16_t* __re
       for (int k = 0; k < NW; ++k) {
         // a wave without a key has l = 0 and sums of 0
         const float mk = sh.g.m[k][qi], lk = sh.g.l[k][qi];
-        const float f = lk == 0.f ? 0.f : (mk == mm ? 1.f : fast_exp2((mk - mm) * c));
+        const float f = lk == 0.f ? 0.f : (mk == mm ? 1.f : expf(mk - mm));
         const float4 x = *reinterpret_cast<const float4*>(&sh.g.o[k][qi * OS + 4 * d4]);
         sum += f * lk;
         o.x += f * x.x, o.y += f * x.y, o.z += f * x.z, o.w += f * x.w;
