@@ -6,7 +6,7 @@ import ctypes
 import pytest
 import torch
 
-from oracle.recurrence import fused_mamba_chunked, fused_mamba_reversed, max_rel
+from oracle.recurrence import fused_mamba_chunked, fused_mamba_reversed, max_rel, rel_fro
 from trifusion_amd import _lib
 from trifusion_amd.mamba_fused import build_args, fused_mamba
 from trifusion_amd.synthetic import clip_inputs
@@ -65,3 +65,29 @@ def test_nan_angle_stays_in_later_rows():
     args[8][0, 200, 0, 5] = float("nan")
     y = fused_mamba(*args)
     assert torch.equal(y[:, :200], clean[:, :200]) and y[0, 200:].isnan().any(-1).all()
+
+
+def serial_walk(dev, out, lengths=None, **kw):
+    """The C entry without a workspace: one workgroup a unit."""
+    a = build_args(*dev, out, lengths, "auto", **kw)
+    assert _lib.load().tf_fused_mamba_workspace_size(ctypes.byref(a)) > 0  # the operator splits this shape
+    _lib.check(_lib.load().tf_fused_mamba(ctypes.byref(a), _lib.stream_of(out)), "fused_mamba")
+    return out
+
+
+def test_phase_of_many_small_steps():
+    """28 800 steps that all turn the same way by ~1e-3 revolutions: the phase sum
+    is held to the fp64 one by the results it moves. With every increment rounded
+    to the nearest 2^-32 revolutions the sum strays by 0.3 sqrt(28 800) units, 7e-8
+    rad, less than the fp32 phase itself, so what remains are q and k elements that
+    round to the other bf16 neighbour, in the segmented form also because it rounds
+    keys in each segment's own phase. Rounding towards 0 would add 2e-5 rad."""
+    args = list(clip_inputs(1, 28800, heads=1, head_dim=64, state=128, rotary=32, seed=3))
+    args[8] = args[8].abs() * 0.02
+    dev = [x.to(DEV) for x in args]
+    out = torch.empty(dev[2].shape, device=DEV)
+    split = fused_mamba(*dev, out=out).cpu()
+    serial = serial_walk(dev, torch.empty_like(out)).cpu()
+    ref = fused_mamba_chunked(*args)
+    print(f"rel_fro segments {rel_fro(split, ref):.3e} serial {rel_fro(serial, ref):.3e}", flush=True)
+    assert rel_fro(split, ref) <= 1.2e-4 and rel_fro(serial, ref) <= 1.2e-4

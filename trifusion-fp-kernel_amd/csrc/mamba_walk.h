@@ -74,11 +74,15 @@ __device__ __forceinline__ PipeItem pipe_item(const MfmaParams& P) {
 
 // Fixed-point phase increment of one (row, pair): pi tanh(theta) dt radians
 // (mamba_fused.py:102-109) = tanh(theta) dt / 2 revolutions, reduced to
-// [-1/2, 1/2] and scaled by 2^32. A row without a step (dt = 0) adds 0.
+// [-1/2, 1/2] and scaled by 2^32. A row without a step (dt = 0) adds 0. NEAREST
+// rounds it to the nearest unit, else towards 0: of increments of one sign that
+// loses half a unit per step, 5e-6 rad over 7200 steps.
+template <bool NEAREST = false>
 __device__ __forceinline__ uint32_t phase_inc(float th, float dt) {
   float om = tanh_fast(th) * dt * 0.5f;
   om -= rintf(om);
-  const float x = fminf(om * 4294967296.f, 2147483520.f);
+  float x = fminf(om * 4294967296.f, 2147483520.f);
+  if constexpr (NEAREST) x = rintf(x);
   return static_cast<uint32_t>(static_cast<int>(x));
 }
 
