@@ -625,13 +625,13 @@ __global__ __launch_bounds__(64) void generic_scan_kernel(const GenericParams<I>
   for (int g0 = 0; g0 < G - 1; g0 += kBatch) {
     float4 d[kBatch];
     double s0[kBatch], s1[kBatch];
-    float m[kBatch];
+    Factor m[kBatch];
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
       const int g = g0 + j;
       if (g < G - 1) {
         d[j] = st[static_cast<int64_t>(g) * kf4];
-        m[j] = exp2f(dec[g]);
+        m[j] = factor_of(dec[g]);
         s0[j] = pair < rot ? ph[g * 64] : 0.0;
         s1[j] = pair + 1 < rot ? ph[g * 64 + 1] : 0.0;
       }
@@ -653,8 +653,9 @@ __global__ __launch_bounds__(64) void generic_scan_kernel(const GenericParams<I>
           x.w = d[j].z * si + d[j].w * co;
         }
         p0 += s0[j], p1 += s1[j];
-        run.x = run.x * m[j] + x.x, run.y = run.y * m[j] + x.y;
-        run.z = run.z * m[j] + x.z, run.w = run.w * m[j] + x.w;
+        const Factor f2 = m[j];
+        run.x = ldexpf(run.x * f2.mant, f2.exp) + x.x, run.y = ldexpf(run.y * f2.mant, f2.exp) + x.y;
+        run.z = ldexpf(run.z * f2.mant, f2.exp) + x.z, run.w = ldexpf(run.w * f2.mant, f2.exp) + x.w;
         st[static_cast<int64_t>(g0 + j) * kf4] = run;
       }
     }

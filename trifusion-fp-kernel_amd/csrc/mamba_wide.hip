@@ -608,13 +608,13 @@ __global__ __launch_bounds__(64) void wide_scan_kernel(const MfmaParams P) {
   uint2 ph = make_uint2(0u, 0u);
   for (int g0 = 0; g0 < G - 1; g0 += kBatch) {
     float4 d[kBatch];
-    float m[kBatch];
+    Factor m[kBatch];
     uint2 s[kBatch];
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) {
       if (g0 + j < G - 1) {
         d[j] = st[static_cast<size_t>(g0 + j) * kRecF4];
-        m[j] = fast_exp2(dec[g0 + j]);
+        m[j] = factor_of(dec[g0 + j]);
         if (turn) s[j] = *reinterpret_cast<const uint2*>(phs + (g0 + j) * RT);
       }
     }
@@ -625,7 +625,9 @@ __global__ __launch_bounds__(64) void wide_scan_kernel(const MfmaParams P) {
           if (g0 + j > 0) d[j] = turn_rows(d[j], ph, rp, R);
           ph = make_uint2(ph.x + s[j].x, ph.y + s[j].y);
         }
-        run = state_step(run, m[j], d[j]);
+        const int e = m[j].exp;
+        run = make_float4(ldexpf(run.x, e), ldexpf(run.y, e), ldexpf(run.z, e), ldexpf(run.w, e));
+        run = state_step(run, m[j].mant, d[j]);
         st[static_cast<size_t>(g0 + j) * kRecF4] = run;
       }
     }

@@ -323,6 +323,19 @@ __device__ __forceinline__ float4 state_step(const float4& s, float m, const flo
                      __builtin_fmaf(s.w, m, d.w));
 }
 
+// 2^x as mant 2^exp, mant in [2^-1/2, 2^1/2], for a factor that may leave the fp32
+// range by itself though the values it is applied to chunk by chunk stay in it (a
+// state of 0, or a small one, over steps that grow). Not a number stays so.
+struct Factor {
+  float mant;
+  int exp;
+};
+__device__ __forceinline__ Factor factor_of(float x) {
+  const float c = x < -600.f ? -600.f : (x > 600.f ? 600.f : x);
+  const float n = rintf(c);
+  return {fast_exp2(c - n), static_cast<int>(n)};
+}
+
 // The segment scan of one unit's records, float4 f of each: record g (the
 // state segment g leaves from zero state; log2 decay dec[g]) is replaced by
 // the state entering segment g: S_0 = 0, S_{g+1} = S_g 2^dec[g] + record g.
