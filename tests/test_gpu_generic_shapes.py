@@ -111,3 +111,23 @@ def test_segments_match_serial_walk(b, t, h, n, p, r, lengths, reverse):
     if lengths is not None:
         for i, length in enumerate(lengths):
             assert not y[i, length:].any()
+
+
+@pytest.mark.parametrize("n", [16, 32])
+def test_infinite_value_gives_infinities(n):
+    """Keys and queries that are all positive and an infinite value: every later
+    output of its head dim is infinite, with the sign of the gate, also where the
+    state dim is padded to a whole tile. Segments turn the states they hand on,
+    which adds infinities of both signs: from the second one on (row 192) the same
+    outputs are not finite, and no others. (The decay of a chunk stays above 0: times
+    infinity that is not a number.)"""
+    q, k, v, adt, dt, trap, qb, kb, angles, d, z = clip_inputs(1, 300, heads=1, head_dim=32, state=n, rotary=n // 4,
+                                                               dtype=torch.float32, seed=n)
+    v[0, 10, 0, 3] = math.inf
+    args = on((q.abs(), k.abs(), v, 0.05 * adt, dt, trap, qb, kb, torch.zeros_like(angles), d, z))
+    expect = math.inf * z[0, 10:, 0, 3].sign()
+    serial, split = call(args, torch.full((1, 300, 1, 32), math.nan, device=DEV)), fused_mamba(*args)
+    assert torch.equal(serial[0, 10:, 0, 3].cpu(), expect)
+    assert torch.equal(split[0, 10:192, 0, 3].cpu(), expect[:182]) and not split[0, 192:, 0, 3].isfinite().any()
+    for y in (serial, split):
+        assert y[..., :3].isfinite().all() and y[..., 4:].isfinite().all() and y[:, :10].isfinite().all()

@@ -288,6 +288,16 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
     }
   };
 
+  // The state copy the products read, channels n0 .. n0 + 3: 0 past the state dim,
+  // where a value that is not finite leaves 0 x infinity, and a query's 0 meets it.
+  auto put_state = [&](int row, int n0, float4 x) {
+    if (n_state < Sm::NP) {
+      x.x = n0 < n_state ? x.x : 0.f, x.y = n0 + 1 < n_state ? x.y : 0.f;
+      x.z = n0 + 2 < n_state ? x.z : 0.f, x.w = n0 + 3 < n_state ? x.w : 0.f;
+    }
+    *reinterpret_cast<float4*>(&sh.st[row * NS + n0]) = x;
+  };
+
   f32x16 state[2] = {zero16(), zero16()};  // state waves
   double carry[RP];             // phase entering the chunk, revolutions
   float seg_log2 = 0.f;
@@ -316,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
           for (int g = 0; g < 4; ++g) {
             const float4 x = rec[(tile * 4 + g) * 64 + ln];
             state[i][4 * g] = x.x, state[i][4 * g + 1] = x.y, state[i][4 * g + 2] = x.z, state[i][4 * g + 3] = x.w;
-            *reinterpret_cast<float4*>(&sh.st[(32 * sp + (ln & 31)) * NS + 32 * sn + 8 * g + 4 * (ln >> 5)]) = x;
+            put_state(32 * sp + (ln & 31), 32 * sn + 8 * g + 4 * (ln >> 5), x);
           }
         }
       }
@@ -565,9 +575,9 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
           for (int e = 0; e < 16; ++e) state[i][e] = state[i][e] * decay + acc[e];
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<float4*>(&sh.st[(32 * sp + c32) * NS + 32 * sn + 8 * g + 4 * hh]) =
-                make_float4(rnd(state[i][4 * g], a.q_dtype), rnd(state[i][4 * g + 1], a.q_dtype),
-                            rnd(state[i][4 * g + 2], a.q_dtype), rnd(state[i][4 * g + 3], a.q_dtype));
+            put_state(32 * sp + c32, 32 * sn + 8 * g + 4 * hh,
+                      make_float4(rnd(state[i][4 * g], a.q_dtype), rnd(state[i][4 * g + 1], a.q_dtype),
+                                  rnd(state[i][4 * g + 2], a.q_dtype), rnd(state[i][4 * g + 3], a.q_dtype)));
         }
       }
     }
@@ -607,7 +617,8 @@ __global__ __launch_bounds__(kThreads) void mamba_generic_kernel(const GenericPa
 // Replaces each unit's segment summaries by the states entering the next
 // segments: S_1 = d_0, S_{g+1} = S_g 2^dec_g + turn_g(d_g), where turn_g rotates
 // the rotary row pairs by the phase entering segment g (a summary is formed from
-// phase 0 at its segment's start, and is linear in the keys that phase turns).
+// phase 0 at its segment's start, and is linear in the keys that phase turns; an
+// infinite element turns into one that is not a number).
 // Thread f of a unit takes float4 f of its records: channels n .. n + 3.
 template <typename I>
 __global__ __launch_bounds__(64) void generic_scan_kernel(const GenericParams<I> P, int kf4, int pt) {
