@@ -3,9 +3,10 @@
 // Same arithmetic and bf16 rounding points as the reference kernel
 // (src/trifusion_l4/mamba_fused.py:72-152), the phase summed in 2^-32 revolutions
 // (increments rounded to nearest). A workgroup of four waves walks one
-// (batch, head) unit, or one time segment of it, in 64-step chunks; two
-// workgroups share a CU (77 KB of LDS and at most 256 registers each), so one's
-// vector work covers the other's latency. Per chunk, between three barriers:
+// (batch, head) unit, or one time segment of it, in 64-step chunks; up to 32 rotary
+// pairs two workgroups share a CU (77 KB of LDS and at most 256 registers each), so
+// one's vector work covers the other's latency (above that the cos/sin table takes
+// 94 KB and one is alone). Per chunk, between three barriers:
 //
 //   rotation   16 rows per wave: [B/C norm,] bias, rotation, scale; values and
 //              decay-scaled values; all to LDS as bf16 rows
@@ -639,10 +640,15 @@ __global__ __launch_bounds__(64) void wide_scan_kernel(const MfmaParams P) {
 // 32 KB, and the phases, in 16 MiB); segments as short as that allows, but of two
 // chunks. The summaries, the scan and their launches pay from six chunks on, from
 // eight above 96 units, and up to 170 units, which leave three segments each (us,
-// split against serial): 64 units, 4 chunks 29.7 / 26.8, 5 40.3 / 34.4, 6 32.2 / 40.8,
-// 29 70.8 / 193; 128 units, 7 chunks 46.3 / 47.0, 8 45.8 / 55.6; 160 units, 7 chunks
-// 51.4 / 48.3, 13 74.3 / 89.6; 192 units in two segments, 13 chunks 96.5 / 89.6.
-constexpr int64_t kGroups = 512, kMaxRecords = 480, kSegment = 2, kMaxUnits = 170;
+// split against serial): 32 units, 6 chunks 30.6 / 40.9, 29 51.4 / 194;
+// 64 units, 4 chunks 29.7 / 26.8, 5 40.3 / 34.4, 6 32.2 / 40.8, 29 70.8 / 193; 128
+// units, 7 chunks 46.3 / 47.0, 8 45.8 / 55.6; 160 units, 7 chunks 51.4 / 48.3, 13
+// 74.3 / 89.6; 192 units in two segments, 13 chunks 96.5 / 89.6.
+// With more than 32 rotary pairs one workgroup fits a CU. One round of them, 256, is
+// the better plan up to 64 units (R 64, 32 units, 29 chunks 63 us against 73 in two
+// rounds); above, too few segments are left and two rounds are (96 units, 29 chunks
+// 162 against 209 serial), up to 128 units (160 units, 13 chunks 124 against 97 serial).
+constexpr int64_t kGroups = 512, kMaxRecords = 480, kSegment = 2, kMaxUnits = 170, kMaxUnits64 = 128;
 
 struct WidePlan {
   int G = 1;
@@ -655,8 +661,10 @@ WidePlan wide_plan(const tf_mamba_args& a) {
   WidePlan p;
   const int64_t units = a.batch * a.heads;
   const int64_t chunks = (a.time + kChunk - 1) / kChunk;
-  if (units <= 0 || units > kMaxUnits || chunks < (units <= 96 ? 6 : 8)) return p;
-  const int64_t g = std::min({kGroups / units, kMaxRecords / units + 1, (chunks + kSegment - 1) / kSegment});
+  const bool table64 = a.rotary > 32;
+  if (units <= 0 || units > (table64 ? kMaxUnits64 : kMaxUnits) || chunks < (units <= 96 ? 6 : 8)) return p;
+  const int64_t groups = table64 && units <= 64 ? kGroups / 2 : kGroups;
+  const int64_t g = std::min({groups / units, kMaxRecords / units + 1, (chunks + kSegment - 1) / kSegment});
   p.G = static_cast<int>(g);
   auto up = [](int64_t x) { return (x + 255) & ~int64_t(255); };
   p.phase_off = up(units * (g - 1) * kRecF4 * 16);
@@ -706,10 +714,14 @@ int launch_wide(const tf_mamba_args& a, hipStream_t stream) {
   const int64_t span = std::max({a.time * a.angles_stride[1], a.time * a.dt_stride[2], a.time * a.adt_stride[2],
                                  a.time * a.trap_stride[2]});
   pieces = pieces && span < (int64_t(1) << 29);
-  if (a.rotary > 32) return launch_wide_kernel<64, 2>(P, stream);
-  if (pieces && !P.ctl_bf16 && !P.trap_bf16 && !ang16) return launch_wide_kernel<32, 0>(P, stream);
-  if (pieces && P.ctl_bf16 && P.trap_bf16 && ang16) return launch_wide_kernel<32, 1>(P, stream);
-  return launch_wide_kernel<32, 2>(P, stream);
+  const bool all32 = pieces && !P.ctl_bf16 && !P.trap_bf16 && !ang16;
+  const bool all16 = pieces && P.ctl_bf16 && P.trap_bf16 && ang16;
+  if (a.rotary > 32) {
+    if (all32) return launch_wide_kernel<64, 0>(P, stream);
+    return all16 ? launch_wide_kernel<64, 1>(P, stream) : launch_wide_kernel<64, 2>(P, stream);
+  }
+  if (all32) return launch_wide_kernel<32, 0>(P, stream);
+  return all16 ? launch_wide_kernel<32, 1>(P, stream) : launch_wide_kernel<32, 2>(P, stream);
 }
 
 }  // namespace tf
