@@ -515,14 +515,50 @@ def launch_depthwise_norm_silu(x, weight, bias, lengths, norm_weight, eps):
 _GATES = {"swiglu": 0, "glu": 1}
 
 
-def gated_linear_fits(x, weight):
+def gated_linear_fits(x, weight, kind):
     """Operands ``tf_gated_linear`` takes, where ``F.linear`` would compute in
-    bf16: bf16 on the device, weight rows contiguous, both widths multiples of
-    64. At every size measured (1 to 28 816 rows) it takes less time than the
-    library's product and the gate kernel after it."""
+    bf16 and the one kernel is the faster way: bf16 on the device, weight rows
+    contiguous, both widths multiples of 64, and sizes that pay."""
     rows, depth = weight.shape
     return (x.is_cuda and x.dtype == weight.dtype == _autocast_dtype(x) == torch.bfloat16 and weight.is_contiguous()
-            and x.shape[-1] == depth and depth % 64 == 0 and rows % 128 == 0 and rows * depth < 2**31)
+            and x.shape[-1] == depth and depth % 64 == 0 and rows % 128 == 0 and 0 < rows * depth < 2**31
+            and gated_linear_pays(x.numel() // depth, rows // 2, depth, kind))
+
+
+def gated_linear_pays(rows, features, depth, kind):
+    """Sizes at which the kernel takes less time than the library's product and the
+    kernel after it (SwiGLU, or for GLU the depthwise one, which gates the rows
+    itself then). The library splits long contractions, which the kernel does not,
+    so with few tiles the line lies by depth and rows x features. Measured, calls in
+    graphs (us, one kernel / two): SwiGLU, depth 512, 1408 features, 16 rows 6.3 / 6.8,
+    6400 rows 27 / 44; depth 1024, 2816 features, 32 rows 8.9 / 8.3, 64 rows 9.3 / 9.6,
+    1616 rows 27 / 38; depth 1536, 101 rows even, 2400 rows 54 / 48; depth 4096, 1024
+    features, one row 25 / 11. Local branch, depth 1024, 1024 features, 101 rows 15.9 /
+    15.1, 160 rows 15.9 / 16.4, 1616 rows 24 / 28; 384 features, 808 rows even; depth
+    512, 128 features, 1024 rows 11.1 / 10.9, 1616 rows 11.8 / 12.6. A grid of 160-row
+    tiles that needs a third round of the CUs is left to the library, up to 1.08 times
+    as fast there at depth 1024. Of 4800 sizes of depth up to 1024 this takes four the
+    slower way by more than 0.5%, by 3% at most."""
+    if type(rows) is not int:  # traced, size unknown
+        return False
+    work = rows * features
+    if kind == "glu":
+        if depth <= 512:
+            return depth <= 128 or work >= 150_000
+        least = 150_000 if features >= 1024 else 400_000
+    else:
+        if depth <= 512:
+            return True
+        least = 150_000
+    if depth > 1024 or work < least:
+        return False
+
+    def rounds(tile):
+        return -(-(-(-rows // tile) * (features // 64)) // 256)
+
+    # the tile that tf_gated_linear takes (linear.hip): least rows and columns fetched
+    tile = min((128, 160, 192), key=lambda t: rounds(t) * (t + 128))
+    return rounds(128) == 1 or tile != 160 or rounds(160) != 3
 
 
 def gated_linear(x, weight, kind):

@@ -105,7 +105,7 @@ class EncoderBlock(nn.Module):
 
     def ffn(self, h):
         g1, g2 = self._padded_rows()
-        if gated_linear_fits(h, g1):
+        if gated_linear_fits(h, g1, "swiglu"):
             return F.linear(gated_linear(h, g1, "swiglu"), g2)
         g1t, g2 = self._padded_ffn()
         return F.linear(swiglu(h @ g1t), g2)

@@ -259,12 +259,12 @@ class Frontend(nn.Module):
         return bands(x).flatten(2), fine, lengths, fine_lengths
 
 
-def _gates(layer, x):
+def _gates(layer, x, kind):
     """Whether ``layer(x)`` and the gate after it run as one ``gated_linear``: a
     plain bias-free layer (no subclass, hook or replaced forward that the
     fused call would pass by) on operands the kernel takes."""
     return (type(layer) is nn.Linear and layer.bias is None and not layer._forward_pre_hooks
-            and not layer._forward_hooks and "forward" not in vars(layer) and gated_linear_fits(x, layer.weight))
+            and not layer._forward_hooks and "forward" not in vars(layer) and gated_linear_fits(x, layer.weight, kind))
 
 
 class LocalCNN(nn.Module):
@@ -385,7 +385,7 @@ class TriFusionBlock(nn.Module):
         """GLU, masked depthwise conv, norm, SiLU, out-projection and the cn
         norm: ``cn``."""
         local = self.local
-        if _gates(local.up, h) and depthwise_norm_silu_fits(h.shape[-1], local.dw):
+        if _gates(local.up, h, "glu") and depthwise_norm_silu_fits(h.shape[-1], local.dw):
             up = gated_linear(h, local.up.weight, "glu")
             return self.cn(local.out(depthwise_norm_silu(up, local.dw, lengths, local.norm)))
         up = local.up(h)
@@ -459,7 +459,10 @@ class TriFusionBlock(nn.Module):
         mn, g = merge_gate(cn, mf, mb, an, self.mn, self.gate)
         merged = self.merge(merge_conv(cn, mn, an, g, self.merge_dw, lengths))
         r, f = add_rms(x, merged, self.ff_norm.weight, None, self.ff_norm.eps, torch.bfloat16)
-        f = gated_linear(f, self.gate_up.weight, "swiglu") if _gates(self.gate_up, f) else swiglu(self.gate_up(f))
+        if _gates(self.gate_up, f, "swiglu"):
+            f = gated_linear(f, self.gate_up.weight, "swiglu")
+        else:
+            f = swiglu(self.gate_up(f))
         down = self.down(f)
         if defer and down.dtype == torch.bfloat16 and block_pre_add_fits(r, down):
             return (r, down), mf, mb
