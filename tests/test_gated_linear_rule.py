@@ -22,3 +22,42 @@ SLOWER = {
 def test_sizes(kind):
     assert all(gated_linear_pays(*s, kind) for s in FASTER[kind])
     assert not any(gated_linear_pays(*s, kind) for s in SLOWER[kind])
+
+
+def test_a_call_that_does_more_than_the_product_is_made(monkeypatch):
+    """Hooks, replaced forwards and subclasses see the layer they were put on."""
+    import torch
+    from torch import nn
+    from torch.nn.modules import module as nn_module
+
+    from trifusion_amd import trifusion
+
+    monkeypatch.setattr(trifusion, "gated_linear_fits", lambda x, weight, kind: True)
+    x = torch.zeros(1, 64)
+
+    def plain():
+        return nn.Linear(64, 128, bias=False)
+
+    assert trifusion._gates(plain(), x, "glu")
+    for register in ("register_forward_hook", "register_forward_pre_hook", "register_full_backward_hook"):
+        layer = plain()
+        getattr(layer, register)(lambda *a: None)
+        assert not trifusion._gates(layer, x, "glu")
+    for register in (nn_module.register_module_forward_hook, nn_module.register_module_forward_pre_hook):
+        handle = register(lambda *a: None)
+        try:
+            assert not trifusion._gates(plain(), x, "glu")
+        finally:
+            handle.remove()
+    layer = plain()
+    layer.forward = lambda x: x
+    assert not trifusion._gates(layer, x, "glu")
+
+    class Weight(torch.Tensor):
+        pass
+
+    layer = plain()
+    layer.weight = nn.Parameter(layer.weight.detach().as_subclass(Weight), requires_grad=False)
+    assert type(layer.weight) is not nn.Parameter and not trifusion._gates(layer, x, "glu")
+    assert not trifusion._gates(nn.Linear(64, 128), x, "glu")
+    assert trifusion._gates(plain(), x, "glu")

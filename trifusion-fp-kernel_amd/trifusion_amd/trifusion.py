@@ -31,6 +31,7 @@ from dataclasses import dataclass
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 from torch.nn.attention import SDPBackend, sdpa_kernel
 
 from .kernels import RMSNorm, gated_concat, swiglu
@@ -261,10 +262,13 @@ class Frontend(nn.Module):
 
 def _gates(layer, x, kind):
     """Whether ``layer(x)`` and the gate after it run as one ``gated_linear``: a
-    plain bias-free layer (no subclass, hook or replaced forward that the
-    fused call would pass by) on operands the kernel takes."""
-    return (type(layer) is nn.Linear and layer.bias is None and not layer._forward_pre_hooks
-            and not layer._forward_hooks and "forward" not in vars(layer) and gated_linear_fits(x, layer.weight, kind))
+    plain bias-free layer whose call would do nothing but ``F.linear`` (no subclass
+    of the layer or its weight, no hook of its own or for all modules, no replaced
+    forward) on operands the kernel takes."""
+    return (type(layer) is nn.Linear and layer.bias is None and type(layer.weight) in (nn.Parameter, torch.Tensor)
+            and not (layer._forward_pre_hooks or layer._forward_hooks or layer._backward_pre_hooks
+                     or layer._backward_hooks or _has_any_global_hook())
+            and "forward" not in vars(layer) and gated_linear_fits(x, layer.weight, kind))
 
 
 class LocalCNN(nn.Module):
