@@ -124,3 +124,24 @@ def test_small_probabilities_are_rounded_once():
     differ = int((y != ref).sum())
     print(f"{differ} of {y.numel()} results not the correctly rounded ones", flush=True)
     assert differ <= 4
+
+
+@pytest.mark.parametrize("b,t", [(1, 65), (1, 129), (20, 256), (20, 257), (64, 768), (64, 800)])
+def test_query_read_on_both_merges(b, t):
+    """Either side of the line between one thread per (query, dim) and eight groups:
+    up to 2 tiles of 64 keys, or one tile for every 40 (head, batch row)s."""
+    g = torch.Generator().manual_seed(b + t)
+    q = torch.randn(10, 256, generator=g).to(BF)
+    kv = torch.randn(b, t, 512, generator=g).to(BF)
+    lengths = torch.randint(0, t + 1, (b,), generator=g)
+    lengths[0] = t
+    y = query_read(q.to(DEV), kv.to(DEV), lengths.to(DEV), 8).cpu().double()
+    k, v = kv.view(b, t, 2, 8, 32).permute(2, 0, 3, 1, 4).unbind(0)
+    qq = q.view(10, 8, 32).transpose(0, 1)[None].expand(b, -1, -1, -1)
+    mask = (torch.arange(t)[None, :] < lengths[:, None])[:, None, None, :]
+    ref = attend(qq, k, v, mask).transpose(1, 2).reshape(b, 10, 256)
+    some = lengths > 0
+    err = (y - ref).abs()[some]
+    # half a bf16 step and fp32 sums of values up to ~5
+    assert (err <= ref.abs()[some] * 2.0**-8 + 5 * 64 * 2.0**-23).all(), err.max()
+    assert not y[~some].any()

@@ -135,6 +135,29 @@ __global__ __launch_bounds__(kMergeGroups * D) void query_read_merge_kernel(cons
   }
 }
 
+// As above, one thread per (query, dim) of one (head, batch row) walking the tiles:
+// for few of them, or more rows than the groups above leave the chip room for.
+template <int NQ, int D>
+__global__ __launch_bounds__(NQ * D) void query_read_merge_few_kernel(const float* __restrict__ part,
+                                                                      uint16_t* __restrict__ y, int H, int S) {
+  constexpr int R = rec_floats<D>(NQ);
+  const int h = blockIdx.x, b = blockIdx.y;
+  const int qi = threadIdx.x / D, d = threadIdx.x - qi * D;
+  const float* base = part + (static_cast<int64_t>(b) * H + h) * S * R + qi * (D + 2);
+  float m = -INFINITY;
+  for (int s = 0; s < S; ++s) m = fmaxf(m, base[static_cast<int64_t>(s) * R]);
+  float l = 0.f, o = 0.f;
+  if (m != -INFINITY) {
+    for (int s = 0; s < S; ++s) {
+      const float* r = base + static_cast<int64_t>(s) * R;
+      const float w = r[0] == -INFINITY ? 0.f : expf(r[0] - m);
+      l += w * r[1];
+      o += w * r[2 + d];
+    }
+  }
+  y[(static_cast<int64_t>(b) * NQ + qi) * H * D + h * D + d] = f32_to_bf16(l > 0.f ? o / l : 0.f);
+}
+
 }  // namespace
 }  // namespace tf
 
@@ -165,6 +188,16 @@ extern "C" int tf_query_read(const void* q, const void* kv, const int64_t* key_l
                      dim3(64), 0, s, static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(kv), key_lengths,
                      part, static_cast<int>(time), static_cast<int>(heads), tiles, scale);
   if (const int rc = tf::launch_status()) return rc;
+  // The whole read, one thread per (query, dim) against eight groups (us, 8 heads): one
+  // row, 2 tiles 12.1 / 12.3, 3 12.8 / 12.4, 32 25.3 / 12.9; 16 rows, 2 tiles 12.8 / 13.1, 4
+  // 14.4 / 13.8; 32 rows, 6 tiles 19.0 / 19.2, 10 41.2 / 40.7; 64 rows, 11 tiles 51.7 /
+  // 54.4, 16 57.4 / 54.1; 128 rows, 16 tiles 89.2 / 90.0, 26 154 / 148.
+  if (tiles <= 2 || 40 * static_cast<int64_t>(tiles) <= batch * heads) {
+    hipLaunchKernelGGL((tf::query_read_merge_few_kernel<10, 32>),
+                       dim3(static_cast<uint32_t>(heads), static_cast<uint32_t>(batch)), dim3(10 * 32), 0, s, part,
+                       static_cast<uint16_t*>(y), static_cast<int>(heads), tiles);
+    return tf::launch_status();
+  }
   hipLaunchKernelGGL((tf::query_read_merge_kernel<10, 32>),
                      dim3(10, static_cast<uint32_t>(heads), static_cast<uint32_t>(batch)),
                      dim3(tf::kMergeGroups * 32), 0, s, part, static_cast<uint16_t*>(y), static_cast<int>(heads), tiles);
