@@ -563,8 +563,13 @@ extern "C" int tf_bands(const void* x, int32_t dtype, const int64_t* strides, vo
   const int64_t total = batch * time * 8 * chans;
   if (total == 0) return TF_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // whole aligned pieces of eight channels
-  const bool vec = strides[1] == 1 && chans % 8 == 0 && strides[0] % 8 == 0 && strides[2] % 8 == 0 &&
+  // Whole aligned pieces of eight channels, where the eighth of the threads still
+  // fills the chip or the loads are long (us, one channel a thread / eight): bf16, 64
+  // channels, 129 frequencies, 25 frames 4.0 / 3.7, 16 x 201 frames 26 / 10; 17
+  // frequencies, 101 frames 2.8 / 3.1; 8 channels, 129 frequencies, 401 frames 3.6 / 4.5
+  // (fp32 3.7 / 6.2).
+  const bool pays = (chans >= 64 && freq >= 64) || (chans >= 16 && batch * time * chans >= 1 << 15);
+  const bool vec = pays && strides[1] == 1 && chans % 8 == 0 && strides[0] % 8 == 0 && strides[2] % 8 == 0 &&
                    strides[3] % 8 == 0 && tf::aligned16(x) && tf::aligned16(y);
   if (vec && (dtype == TF_FLOAT32 || dtype == TF_BFLOAT16)) {
     auto launch = [&](auto* p) {
