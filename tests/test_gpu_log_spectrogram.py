@@ -47,3 +47,11 @@ def test_bands_by_pieces(b, t, f, c, dtype):
     x = torch.randn(b, t, f, c, generator=torch.Generator().manual_seed(f)).to(dtype).to(DEV)
     y = bands(x.permute(0, 3, 1, 2))  # channels last: pieces of eight
     assert torch.equal(y, bands(x.permute(0, 3, 1, 2).contiguous()))
+
+
+def test_short_lengths_are_refused():
+    audio, window = torch.zeros(4, 1, 400, device=DEV), torch.ones(400, device=DEV)
+    whole, short = torch.full((4,), 400, device=DEV), torch.full((3,), 1, device=DEV)
+    for lengths, channels in ((short, whole), (whole, short)):
+        with pytest.raises(ValueError, match="entry per clip"):
+            log_spectrogram(audio, window, lengths, channels)

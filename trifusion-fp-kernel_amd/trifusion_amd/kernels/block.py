@@ -776,6 +776,8 @@ def launch_log_spectrogram(audio, window, lengths, channels):
         raise ValueError("log_spectrogram: audio must be [B, C, N] and the window [400]")
     x = audio.float().contiguous()
     b, c, n = x.shape
+    if lengths.numel() < b or channels.numel() < b:  # read per clip
+        raise ValueError("log_spectrogram: lengths and channels must have an entry per clip")
     y = torch.empty((b, n // 160 + 1, 257), device=x.device, dtype=torch.float32)
     status = lib.tf_log_spectrogram(x.data_ptr(), window.float().contiguous().data_ptr(), _lengths(lengths).data_ptr(),
                                     _lengths(channels).data_ptr(), y.data_ptr(), b, c, n, _lib.stream_of(x))
