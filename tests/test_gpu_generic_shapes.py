@@ -131,3 +131,31 @@ def test_infinite_value_gives_infinities(n):
     assert torch.equal(split[0, 10:192, 0, 3].cpu(), expect[:182]) and not split[0, 192:, 0, 3].isfinite().any()
     for y in (serial, split):
         assert y[..., :3].isfinite().all() and y[..., 4:].isfinite().all() and y[:, :10].isfinite().all()
+
+
+@pytest.mark.parametrize("at", [10, 300, 630])
+@pytest.mark.parametrize("bad", [math.inf, math.nan])
+def test_value_that_is_not_finite_in_segments(at, bad):
+    """In segments (640 rows of one unit: five of two chunks) a row of v that is not
+    finite leaves earlier rows and other head dims as they were, and no later output
+    of its own is finite."""
+    args = on(clip_inputs(1, 640, heads=1, head_dim=64, state=64, dtype=torch.float32, seed=9))
+    clean = fused_mamba(*args)
+    v = args[2].clone()
+    v[0, at, 0, 3] = bad
+    y = fused_mamba(*args[:2], v, *args[3:])
+    assert max_rel(y[:, :at].cpu(), clean[:, :at].cpu()) <= 5e-6
+    assert not y[0, at:, 0, 3].isfinite().any()
+    rest = [i for i in range(64) if i != 3]
+    assert max_rel(y[..., rest].cpu(), clean[..., rest].cpu()) <= 5e-6
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+def test_positive_decay_in_segments(reverse):
+    """A fifth of the steps grow, in segments, against the fp32 oracle."""
+    args = list(clip_inputs(1, 900, heads=4, head_dim=64, state=64, dtype=torch.float32, seed=44))
+    flip = torch.rand(args[3].shape, generator=torch.Generator().manual_seed(1)) < 0.2
+    args[3] = torch.where(flip, -0.25 * args[3], args[3])
+    y = fused_mamba(*on(args), reverse=reverse)
+    ref = (fused_mamba_reversed if reverse else fused_mamba_chunked)(*args)
+    assert max_rel(y.cpu(), ref) <= 1e-5

@@ -73,7 +73,7 @@ def test_positive_decay_steps_match_oracle(case, variant, reverse):
     out = torch.empty(dargs[2].shape, device=DEV, dtype=torch.float32)
     if segmented:
         if variant == "generic":
-            pytest.skip("the generic kernel has no chunk-parallel form")
+            pytest.skip("the generic kernel has a chunk-parallel form for fp32 operands only")
         assert _workspace_bytes(dargs, out, variant) > 0, "shape does not take the chunk-parallel path"
     print(f"case {case} variant={variant} reverse={reverse}", flush=True)
     with torch.inference_mode():

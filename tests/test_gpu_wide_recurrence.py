@@ -6,6 +6,7 @@ import ctypes
 import pytest
 import torch
 
+from oracle.elementwise import mamba_controls, rms_norm
 from oracle.recurrence import fused_mamba_chunked, fused_mamba_reversed, max_rel, rel_fro
 from trifusion_amd import _lib
 from trifusion_amd.mamba_fused import build_args, fused_mamba
@@ -24,8 +25,8 @@ def padded(x, before, after):
 
 
 # rotary: a full table of 32, above it (64 rows of table), not a multiple of 8,
-# none in the last piece; angles: aligned pieces or single elements; controls fp32
-# or (as the model's raw projection) bf16; q/k/v/z rows 16- or 8-byte aligned
+# none in the last piece; angles: aligned pieces or single elements; fp32 controls
+# (test_model_form has the model's raw bf16 ones); q/k/v/z rows 16- or 8-byte aligned
 @pytest.mark.parametrize("rotary", [32, 64, 33, 9, 1])
 @pytest.mark.parametrize("form", ["fp32", "bf16", "odd"])
 @pytest.mark.parametrize("reverse", [False, True])
@@ -34,7 +35,7 @@ def test_forms_and_edges(rotary, form, reverse):
     b, t, h = len(lens), 400, 2
     print(f"case rotary={rotary} form={form} reverse={reverse}", flush=True)
     args = list(clip_inputs(b, t, heads=h, head_dim=64, state=128, rotary=rotary, seed=rotary))
-    if form == "bf16":  # trapezoid and angles bf16; raw bf16 controls are the model's own tests
+    if form == "bf16":  # trapezoid and angles bf16 beside fp32 controls: read element by element
         args[5], args[8] = args[5].to(torch.bfloat16), args[8].to(torch.bfloat16)
     dev = [x.to(DEV) for x in args]
     if form == "odd":
@@ -91,3 +92,80 @@ def test_phase_of_many_small_steps():
     ref = fused_mamba_chunked(*args)
     print(f"rel_fro segments {rel_fro(split, ref):.3e} serial {rel_fro(serial, ref):.3e}", flush=True)
     assert rel_fro(split, ref) <= 1.2e-4 and rel_fro(serial, ref) <= 1.2e-4
+
+
+def model_operands(b, t, h, rotary, seed):
+    """What a Mamba layer's projection hands the recurrence: columns [z | v | k | q |
+    ddt | a | trap | angles] of one bf16 buffer, the angles shared by all heads, with
+    an fp32 step bias and B/C norm weights. The kernel's packed form reads them."""
+    g = torch.Generator().manual_seed(seed)
+    n, p = 128, 64
+    x = torch.randn(b, t, 2 * h * p + 2 * n + 3 * h + rotary, generator=g)
+    x[..., -rotary:] *= 0.3
+    x = x.to(torch.bfloat16).to(DEV)
+    z, v, k, q, ddt, a, trap, angles = x.split([h * p, h * p, n, n, h, h, h, rotary], -1)
+    assert angles.data_ptr() % 16 == 0 and x.shape[-1] % 8 == 0 and rotary % 8 == 0  # pieces of eight angles
+    qb, kb = (1 + 0.1 * torch.randn(h, n, generator=g) for _ in range(2))
+    wq, wk = (0.5 + torch.rand(n, generator=g) for _ in range(2))
+    bias, d = torch.randn(h, generator=g) - 4, torch.ones(h)
+    args = (q.unsqueeze(2), k.unsqueeze(2), v.unflatten(-1, (h, p)), a.transpose(1, 2), ddt.transpose(1, 2),
+            trap.transpose(1, 2), qb.to(DEV), kb.to(DEV), angles.unsqueeze(2).expand(-1, -1, h, -1), d.to(DEV),
+            z.unflatten(-1, (h, p)))
+    kw = dict(dt_bias=bias.to(DEV), a_floor=1e-4, q_norm=wq.to(DEV), k_norm=wk.to(DEV), norm_eps=1e-5)
+    adt, dt = mamba_controls(a.cpu(), ddt.cpu(), bias, 1e-4)
+    ref = [x.cpu() for x in args]
+    ref[0], ref[1], ref[3], ref[4] = rms_norm(ref[0], wq, 1e-5), rms_norm(ref[1], wk, 1e-5), adt, dt
+    return args, kw, ref
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("rotary", [32, 64, 24])
+@pytest.mark.parametrize("b,t,h,lens", [(24, 130, 8, "ragged"), (2, 700, 8, (700, 333)), (1, 1300, 16, None)])
+def test_model_form(b, t, h, lens, rotary, reverse):
+    """Raw bf16 controls, bf16 trapezoid and angles and fused norms, as every layer of
+    the models passes them: 192 units of up to three chunks in one walk each, and few
+    units in segments, against the oracle and the serial walk. Where the norm, the
+    rotation or the phase differs in its last fp32 bit, a q or k element near the
+    middle of two bf16 values rounds to the other one: 2^-8 of that element, so of one
+    term of a result (no larger than the largest result), for one element in some 2^13
+    (2^-22 against a step of 2^-8, both sides), which is 2^-8 2^-6.5 = 4e-5 of the
+    norm; five times that is allowed. Segments round every key in another frame than
+    the oracle: two roundings of a key, 2^-9 / sqrt(3) of it at most in root mean
+    square, differ by 1.6e-3 of it, and so does what a state hands on, part of a
+    result (2e-4 here)."""
+    print(f"case B{b} T{t} H{h} R{rotary} reverse={reverse}", flush=True)
+    args, kw, ref = model_operands(b, t, h, rotary, seed=b + rotary)
+    if lens == "ragged":
+        lens = [(37 * i) % (t + 1) for i in range(b - 1)] + [t]
+    lengths = None if lens is None else torch.tensor(lens)
+    dl = None if lengths is None else lengths.to(DEV)
+    out = torch.full((b, t, h, 64), float("nan"), device=DEV)
+    y = fused_mamba(*args, out=out, lengths=dl, reverse=reverse, **kw).cpu()
+    expect = (fused_mamba_reversed if reverse else fused_mamba_chunked)(*ref, lengths=lengths)
+    split = b * h <= 128
+    got = [(y, 1.6e-3 if split else 2e-4)]
+    if split:
+        got.append((serial_walk(args, torch.full_like(out, float("nan")), dl, reverse=reverse, **kw).cpu(), 2e-4))
+    for x, bound in got:
+        print(f"  max_rel {max_rel(x, expect):.3e} rel_fro {rel_fro(x, expect):.3e}", flush=True)
+        assert max_rel(x, expect) <= 2.0**-8 and rel_fro(x, expect) <= bound
+    for i, length in enumerate(lens or ()):
+        assert not y[i, length:].any()
+
+
+@pytest.mark.parametrize("reverse", [False, True])
+@pytest.mark.parametrize("b,t,h", [(24, 130, 8), (1, 700, 8)])
+def test_positive_decay(b, t, h, reverse):
+    """A fifth of the steps grow: scores are capped at weight 1 inside a chunk, the
+    carried state is not (as tests/test_gpu_positive_decay.py has it for N = 64)."""
+    args = list(clip_inputs(b, t, heads=h, head_dim=64, state=128, rotary=32, seed=43))
+    flip = torch.rand(args[3].shape, generator=torch.Generator().manual_seed(1)) < 0.2
+    args[3] = torch.where(flip, -0.25 * args[3], args[3])
+    out = torch.empty(b, t, h, 64, device=DEV)
+    dev = [x.to(DEV) for x in args]
+    got = [fused_mamba(*dev, out=out, reverse=reverse)]
+    if b == 1:
+        got.append(serial_walk(dev, torch.empty_like(out), reverse=reverse))
+    ref = (fused_mamba_reversed if reverse else fused_mamba_chunked)(*args)
+    for y in got:
+        assert y.isfinite().all() and max_rel(y.cpu(), ref) <= MAX_REL
