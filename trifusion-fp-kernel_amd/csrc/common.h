@@ -12,7 +12,6 @@ namespace tf {
 
 constexpr float kLog2e = 1.44269504089f;  // rounded log2(e) the recurrence scales adt by
 constexpr float kPi = 3.141592653589793f;
-constexpr float kTwoPi = 6.283185307179586f;
 constexpr float kInvTwoPi = 0.15915494309189535f;
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
@@ -97,33 +96,12 @@ __device__ __forceinline__ float softplus_le20(float v) {
   return v < -104.f ? 0.f : (u == 1.f ? x : r);
 }
 
-// x - 2pi*floor(x/2pi), the reduction the reference applies to phases.
-__device__ __forceinline__ float mod_two_pi(float x) {
-  return x - kTwoPi * floorf(x / kTwoPi);
-}
-
-constexpr double kPiD = 3.141592653589793;
 constexpr double kTwoPiD = 6.283185307179586;
-
-__device__ __forceinline__ double mod_two_pi_d(double x) {
-  return x - kTwoPiD * floor(x / kTwoPiD);
-}
 
 // Wave64 sum via xor shuffles (every lane receives the total).
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-// Inclusive prefix sum across the 64 lanes of a wave (Hillis-Steele).
-__device__ __forceinline__ float wave_inclusive_scan(float v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    float o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
-  }
   return v;
 }
 
