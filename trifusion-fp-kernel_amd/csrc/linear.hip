@@ -18,8 +18,11 @@
 // and the 64-row tile (three stages) is for grids that do not fill the chip. SwiGLU
 // layer, against the library's product and a gate kernel: 6400 x (2 x 1408) x 512
 // 41.2 -> 25.8 us, 1616 x (2 x 2816) x 1024 36.0 -> 27.3, 404 rows 17.5 -> 11.3,
-// 28 816 rows 364 -> 334; one row of 64 6.1 -> 2.9. GLU, 1616 x (2 x 1024) x 1024: 13.2 us against 12.3 for the library's product
-// alone, and the convolution after it 12.4 -> 8.0 on rows that are gated once.
+// 28 816 rows 364 -> 334; one row of 64 6.1 -> 2.9. GLU, 1616 x (2 x 1024) x 1024: 13.2
+// us against 12.3 for the library's product alone, and the convolution after it 12.4 ->
+// 8.0 on rows that are gated once (in the model, beside the attention branch, 20.1
+// against 16.5 and 15.8 -> 9.9). Long contractions are not split over workgroups: with
+// few tiles and much depth the library is faster, and the callers leave those to it.
 #include <algorithm>
 
 #include "mfma_tile.h"

@@ -991,7 +991,7 @@ bool mfma_supported(const tf_mamba_args& a) {
 // chunks (four waves, one per SIMD): its working set needs the 512 registers a
 // lone wave gets. N=128, P=64 runs on mamba_wide.hip at every size: 512 units of
 // 101 rows took 38.6 us here and take 21.0 there, 32 units of 1801 rows 92.3 and
-// 49.9.
+// 49.9; with 64 rotary pairs 45.5 and 39.9, 113 and 73.
 int launch_mfma(const tf_mamba_args& a, hipStream_t stream) {
   const int nt = static_cast<int>(padded_state(a) / 32);
   const int pt = static_cast<int>(a.head_dim / 32);
